@@ -1842,6 +1842,27 @@ template <typename T> struct Stepper : public StepperBase {
         MM_HIP(hipMemcpy(ctl, &c, sizeof(c), hipMemcpyHostToDevice));
     }
 
+    // Attempts worth enqueueing before the next look at the control block of a
+    // run with an end or stop time: those that reach it at the present step
+    // size, and for an end time the clipped one that follows the step past it.
+    // What is enqueued beyond the stop costs the field passes of whole
+    // attempts, since only the stage and control kernels look at the stop
+    // flag; a look costs some 20 us.  Measured on MI355X: 1 ps of the
+    // 150x90x14 FP32 block (20 steps) 21.0 ms with a fixed 64 attempts per
+    // look, 9.8 ms with this count; the 1024x1024x2 film's 67.7 -> 25.5 ms.
+    static long long attempts_left(const StepCtl &c)
+    {
+        long long q = 1ll << 40;
+        if (!(c.h > 0.0)) return q;
+        auto reach = [&](double t_to, long long more) {
+            const double r = (t_to - c.t) / c.h;
+            if (r < 1e9) q = std::min(q, (long long)std::max(r, 0.0) + more);
+        };
+        if (c.tmax_on) reach(c.t_max, c.forced ? 0 : 2);
+        if (c.tstop_on) reach(c.t_stop, 1);
+        return q;
+    }
+
     // enqueue attempts in batches until the device sets stop; c holds the
     // control block on entry (already on the device) and on return
     void drive(StepCtl &c, long long batch)
@@ -1854,8 +1875,11 @@ template <typename T> struct Stepper : public StepperBase {
             MM_HIP(hipStreamSynchronize(s));
             MM_HIP(hipMemcpy(&c, ctl, sizeof(c), hipMemcpyDeviceToHost));
         }
-        while (!c.stop) {
-            const long long q = std::max(1ll, std::min(batch, c.target - c.accepted));
+        // with an end time the batches start at 8 and double, since a step size
+        // that is still growing says little about the attempts to come
+        const bool timed = c.tmax_on || c.tstop_on;
+        for (long long cap = timed ? 8 : batch; !c.stop; cap = std::min(batch, 2 * cap)) {
+            const long long q = std::max(1ll, std::min(std::min(cap, c.target - c.accepted), attempts_left(c)));
             launch_attempts(q);
             MM_HIP(hipStreamSynchronize(s));
             MM_HIP(hipMemcpy(&c, ctl, sizeof(c), hipMemcpyDeviceToHost));
