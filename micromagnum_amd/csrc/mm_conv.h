@@ -4,6 +4,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <cstdlib>
 #include <type_traits>
 #include <vector>
 
@@ -87,6 +88,68 @@ struct ConvLaunch {
     int tk_y;   // kx columns per WG, y passes
     int tk_z;   // kx columns per WG, z pass (3 components each)
 };
+
+// End of the x forward passes: the lpw lines of workgroup blk (two real rows
+// per complex line, transformed in LDS) as half spectra
+// X0[k] = (Z[k] + conj Z[L-k]) / 2, X1[k] = (Z[k] - conj Z[L-k]) / 2i.
+// row(h): where row h of the nrows rows goes.  Short spectra take several
+// lines at a time; the thread of k = 0 also writes k = L/2 of an even line.
+template <typename T, typename ROW>
+__device__ __forceinline__ void xfwd_store(const C2<T> *sm, int LP, int L, int lpw, int blk, int nrows, int Hx,
+                                           ROW row)
+{
+    constexpr int SK = MM_SKEW_X;
+    const int nt = (int)blockDim.x, t = (int)threadIdx.x;
+    const int kh = (L & 1) ? Hx : Hx - 1;
+    const int ng = max(1, nt / kh), g = ng == 1 ? 0 : t / kh;
+    for (int l2 = g < ng ? g : lpw; l2 < lpw; l2 += ng) {
+        const int h0 = 2 * (blk * lpw + l2);
+        if (h0 >= nrows) break;
+        const C2<T> *ln = sm + (size_t)l2 * LP;
+        C2<T> *d0 = row(h0), *d1 = h0 + 1 < nrows ? row(h0 + 1) : nullptr;
+        for (int k = t - g * kh; k < kh; k += ng == 1 ? nt : kh) {
+            const C2<T> zk = ln[sk<SK>(k)], zm = ln[sk<SK>(k == 0 ? 0 : L - k)];
+            d0[k] = cmk<T>((zk.x + zm.x) * (T)0.5, (zk.y - zm.y) * (T)0.5);
+            if (d1) d1[k] = cmk<T>((zk.y + zm.y) * (T)0.5, (zm.x - zk.x) * (T)0.5);
+            if (k == 0 && kh < Hx) {
+                const C2<T> zh = ln[sk<SK>(kh)];
+                d0[kh] = cmk<T>(zh.x, (T)0);
+                if (d1) d1[kh] = cmk<T>(zh.y, (T)0);
+            }
+        }
+    }
+}
+
+// multiplier for udiv: n / d for every n < nmax (0: not exact, divide;
+// wide: always divide)
+static inline unsigned mdiv(unsigned d, size_t nmax, bool wide = false)
+{
+    MM_REQUIRE(d >= 1, "zero divisor");
+    if (d == 1 || (unsigned long long)nmax * d >= (1ull << 32) || wide) return 0u;
+    return (unsigned)((1ull << 32) / d + 1);
+}
+
+static inline int floor_pow2(int v) { return v < 1 ? 1 : 1 << (31 - __builtin_clz((unsigned)v)); }
+
+static inline int env_int(const char *name, int dflt)
+{
+    const char *v = std::getenv(name);
+    return (v && *v) ? std::atoi(v) : dflt;
+}
+
+// LDS bytes of `nlines` transform lines of length L plus the plan's twiddle table
+template <int SK> inline size_t lines_lds(int nlines, int L, size_t csize)
+{
+    return ((size_t)nlines * lds_len<SK>(L) + (size_t)L) * csize;
+}
+
+// Launch shapes: x passes take several rows per workgroup; the strided y and
+// z passes take tiles of adjacent kx columns (row segments of tile*16 or
+// tile*8 bytes).  Tiles are sized for several resident workgroups per CU so
+// that global loads of one overlap the FFT of another.  MM_LPW_X, MM_TK_Y and
+// MM_TK_Z override the choice (launch-shape sweeps).
+ConvLaunch mm_choose_launch(const ConvGeom &g, const FftPlanHost &px, const FftPlanHost &py, const FftPlanHost &pz,
+                            size_t csize);
 
 // Optional per-launch event log used by the measurement entry point: after
 // every kernel the owner records an event tagged with the kernel class.
