@@ -28,7 +28,23 @@ struct FftPlanHost {
     void *twp32 = nullptr; // float2[ntw], per-pass layout (FftPlanDev)
     void *twp64 = nullptr; // double2[ntw]
     int ntw = 0;
+    int id = 0;             // compiled plan (mm_plan_id), 0: none
     void build(int len);
+    // the plan as kernels that run the passes in a loop take it (the same
+    // passes and twiddles, L/8 threads per line)
+    static int tline_loop(int len) { return len > MM_FFT_EPT ? (len + MM_FFT_EPT - 1) / MM_FFT_EPT : 1; }
+    void no_compiled()
+    {
+        id = 0;
+        tline = tline_loop(L);
+    }
+    template <typename T> FftPlanDev dev_loop() const
+    {
+        FftPlanDev d = dev<T>();
+        d.tline = tline_loop(L);
+        d.id = 0;
+        return d;
+    }
     void release();
     template <typename T> FftPlanDev dev() const
     {
@@ -41,35 +57,29 @@ struct FftPlanHost {
         d.tw = sizeof(T) == 4 ? twp32 : twp64;
         d.ntw = ntw;
         d.pow2 = (L & (L - 1)) == 0 ? 1 : 0;
+        d.id = id;
         return d;
     }
     // the plain table exp(-2 pi i m / L), m < L
     template <typename T> const void *plain() const { return sizeof(T) == 4 ? tw32 : tw64; }
 };
 
-// Calls f(std::integral_constant<int, LC>()) with LC = L when kernels carry a
-// compile-time plan for that length (powers of two 2..2048) and `generic` is
-// false, else LC = 0 (runtime plan).
-template <typename F> void mm_with_len(int L, bool generic, F &&f)
+// Calls f(std::integral_constant<int, LC>()) with the kernel instantiation for
+// lines of length L: LC = L for powers of two 2..2048 (unless `generic`),
+// MM_LC_ANY (MM_LC_Z for the z pass) for the other compiled lengths, else 0,
+// the runtime plan.
+template <int ANY = MM_LC_ANY, typename F> void mm_with_len(int L, bool generic, F &&f)
 {
-    if (generic) {
-        f(std::integral_constant<int, 0>());
-        return;
+    if (!generic) {
+        switch (L) {
+#define MM_FFT_X(N) case N: f(std::integral_constant<int, N>()); return;
+        MM_FFT_POW2(MM_FFT_X)
+#undef MM_FFT_X
+        default: break;
+        }
     }
-    switch (L) {
-    case 2: f(std::integral_constant<int, 2>()); return;
-    case 4: f(std::integral_constant<int, 4>()); return;
-    case 8: f(std::integral_constant<int, 8>()); return;
-    case 16: f(std::integral_constant<int, 16>()); return;
-    case 32: f(std::integral_constant<int, 32>()); return;
-    case 64: f(std::integral_constant<int, 64>()); return;
-    case 128: f(std::integral_constant<int, 128>()); return;
-    case 256: f(std::integral_constant<int, 256>()); return;
-    case 512: f(std::integral_constant<int, 512>()); return;
-    case 1024: f(std::integral_constant<int, 1024>()); return;
-    case 2048: f(std::integral_constant<int, 2048>()); return;
-    default: f(std::integral_constant<int, 0>()); return;
-    }
+    if (mm_plan_id(L) > 0 && (ANY != MM_LC_Z || mm_plan_z(L))) f(std::integral_constant<int, ANY>());
+    else f(std::integral_constant<int, 0>());
 }
 
 bool mm_is_smooth(int n);                  // n has no prime factor > 5
@@ -189,8 +199,9 @@ struct KernelLog {
 // Each system of a batch has a descriptor per pass; the launch's global
 // workgroup g (in XCD order, xcd_tile) belongs to system tsys[g] and is that
 // system's workgroup g - tbase.  A system whose stop flag is set skips the
-// pass.  Lengths differ between systems, so the transforms take the runtime
-// FFT plans.
+// pass.  Lengths differ between systems, so each workgroup selects its
+// system's compiled plan (or all run the runtime plans, if one has no such
+// length).
 template <typename T> struct BxDesc {  // x forward of the current state y[*sel]
     const T *y0, *y1;
     const int *sel, *stop;
@@ -233,6 +244,7 @@ struct BatchPass {
     int ntiles = 0, threads = 0;
     size_t lds = 0;
     bool o32 = true;
+    bool compiled = true;  // every system's lines have a compiled length
 };
 
 template <typename T>

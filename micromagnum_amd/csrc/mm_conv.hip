@@ -21,18 +21,13 @@ void FftPlanHost::build(int len)
 {
     MM_REQUIRE(len >= 1, "FFT length must be positive");
     L = len;
-    rad.clear();
-    int n = len;
-    int twos = 0;
-    while (n % 2 == 0) { n /= 2; ++twos; }
-    while (twos >= 3) { rad.push_back(8); twos -= 3; }
-    if (twos == 2) rad.push_back(4);
-    if (twos == 1) rad.push_back(2);
-    while (n % 5 == 0) { rad.push_back(5); n /= 5; }
-    while (n % 3 == 0) { rad.push_back(3); n /= 3; }
-    if (n != 1) throw mm_error(MM_ERR_UNSUPPORTED, "FFT length " + std::to_string(len) + " has a prime factor > 5");
-    MM_REQUIRE(rad.size() <= MM_FFT_MAX_PASSES, "FFT length needs too many passes");
-    tline = std::max(1, (L + MM_FFT_EPT - 1) / MM_FFT_EPT);
+    const FftRadices f = mm_plan_radices(len);
+    if (f.n == 0 && len != 1)
+        throw mm_error(MM_ERR_UNSUPPORTED, "FFT length " + std::to_string(len) + " has a prime factor > 5");
+    MM_REQUIRE(f.n <= MM_FFT_MAX_PASSES, "FFT length needs too many passes");
+    rad.assign(f.r, f.r + f.n);
+    id = mm_plan_id(len);
+    tline = id > 0 ? mm_plan_tline(len) : tline_loop(len);
     if (tline > 1024) throw mm_error(MM_ERR_UNSUPPORTED, "FFT length " + std::to_string(len) + " above 8192");
     std::vector<float2> t32(L);
     std::vector<double2> t64(L);

@@ -589,6 +589,7 @@ void ConvImpl<T>::init(const double *N_host, int nx, int ny, int nz, int ex, int
     px.build(g.Px);
     py.build(g.Py);
     pz.build(g.Pz);
+    if (!mm_plan_z(g.Pz)) pz.no_compiled();
     ln = mm_choose_launch(g, px, py, pz, sizeof(C2<T>));
     // MM_FFT_GENERIC=1: runtime FFT plans for every length (tests compare
     // them with the compile-time plans)
@@ -611,6 +612,7 @@ void ConvImpl<T>::init(const double *N_host, int nx, int ny, int nz, int ex, int
         prune_y = want && !g.is2d && g.Py % 2 == 0 && ny <= g.Py / 2 && g.Py / 2 >= 8;
         if (prune_y) {
             pyh.build(g.Py / 2);
+            pyh.no_compiled();
             const int lds = mm_max_lds_bytes();
             const size_t cs = sizeof(C2<T>);
             int tk = env_int("MM_TK_YP", (int)(128 / cs));
@@ -657,15 +659,15 @@ void ConvImpl<T>::init(const double *N_host, int nx, int ny, int nz, int ex, int
     MM_HIP(hipMalloc(&T1, sizeof(double2) * nspec));
     MM_HIP(hipMalloc(&T2, sizeof(double2) * nspec));
     const int lds = mm_max_lds_bytes();
-    const FftPlanDev dx = px.dev<double>(), dy = py.dev<double>(), dz = pz.dev<double>();
-    int lpw = std::max(1, 256 / px.tline);
-    while (lpw > 1 && lines_lds<MM_SKEW_X>(lpw, px.L, 16) > (size_t)lds) --lpw;
+    const FftPlanDev dx = px.dev_loop<double>(), dy = py.dev_loop<double>(), dz = pz.dev_loop<double>();
+    int lpw = std::max(1, 256 / dx.tline);
+    while (lpw > 1 && lines_lds<MM_SKEW_X>(lpw, dx.L, 16) > (size_t)lds) --lpw;
     int tky = 8;
-    while (tky > 1 && ((size_t)tky * py.tline > 1024 || lines_lds<MM_SKEW_Y>(tky, py.L, 16) > (size_t)lds)) tky /= 2;
+    while (tky > 1 && ((size_t)tky * dy.tline > 1024 || lines_lds<MM_SKEW_Y>(tky, dy.L, 16) > (size_t)lds)) tky /= 2;
     int tkz = 8;
-    while (tkz > 1 && ((size_t)tkz * pz.tline > 1024 || lines_lds<MM_SKEW_Z>(tkz, pz.L, 16) > (size_t)lds)) tkz /= 2;
-    const size_t shx = lines_lds<MM_SKEW_X>(lpw, px.L, 16), shy = lines_lds<MM_SKEW_Y>(tky, py.L, 16),
-                 shz = lines_lds<MM_SKEW_Z>(tkz, pz.L, 16);
+    while (tkz > 1 && ((size_t)tkz * dz.tline > 1024 || lines_lds<MM_SKEW_Z>(tkz, dz.L, 16) > (size_t)lds)) tkz /= 2;
+    const size_t shx = lines_lds<MM_SKEW_X>(lpw, dx.L, 16), shy = lines_lds<MM_SKEW_Y>(tky, dy.L, 16),
+                 shz = lines_lds<MM_SKEW_Z>(tkz, dz.L, 16);
     set_lds(k_xfwd<double, double>, shx);
     set_lds(k_yfwd<double>, shy);
     set_lds(k_zfwd_setup, shz);
@@ -673,16 +675,16 @@ void ConvImpl<T>::init(const double *N_host, int nx, int ny, int nz, int ex, int
     for (int e = 0; e < 6; ++e) {
         MM_HIP(hipMemcpy(dN, Nr.data() + e * plane_full, sizeof(double) * plane_full, hipMemcpyHostToDevice));
         const int nrows = Py * Pz;
-        hipLaunchKernelGGL((k_xfwd<double, double>), dim3(((nrows + 1) / 2 + lpw - 1) / lpw), dim3(lpw * px.tline), shx, 0,
+        hipLaunchKernelGGL((k_xfwd<double, double>), dim3(((nrows + 1) / 2 + lpw - 1) / lpw), dim3(lpw * dx.tline), shx, 0,
                            dN, 0, T1, 0, g.Hx, g.Hp, Py, Pz, nrows, Px, dx, lpw, (const double *)nullptr,
                            (const int *)nullptr);
         MM_HIP(hipGetLastError());
         const unsigned ntyk = (unsigned)((g.Hx + tky - 1) / tky), nbk = ntyk * Pz;
-        hipLaunchKernelGGL((k_yfwd<double>), dim3(ntyk, Pz, 1), dim3(tky * py.tline), shy, 0, T1, T2, g.Hx, g.Hp, Py,
+        hipLaunchKernelGGL((k_yfwd<double>), dim3(ntyk, Pz, 1), dim3(tky * dy.tline), shy, 0, T1, T2, g.Hx, g.Hp, Py,
                            Pz, dy, tky, 0, mdiv(ntyk, nbk), mdiv((unsigned)Pz, nbk));
         MM_HIP(hipGetLastError());
         if (Pz > 1) {
-            hipLaunchKernelGGL(k_zfwd_setup, dim3((g.Hx + tkz - 1) / tkz, Py, 1), dim3(tkz * pz.tline), shz, 0,
+            hipLaunchKernelGGL(k_zfwd_setup, dim3((g.Hx + tkz - 1) / tkz, Py, 1), dim3(tkz * dz.tline), shz, 0,
                                T2, g.Hx, g.Hp, Py, dz, tkz);
             MM_HIP(hipGetLastError());
         }
@@ -803,7 +805,7 @@ template <typename T> void ConvImpl<T>::spectral(hipStream_t s)
     const size_t zsb = (size_t)g.Py * g.Hp * cs;
     const bool o32 = zsb < (1u << 24) && 3 * (size_t)g.nz * zsb < (1ull << 32) &&
                      kern_elems * sizeof(T) < (1ull << 32) && !wide;
-    mm_with_len(pz.L, fft_generic, [&](auto lc) {
+    mm_with_len<MM_LC_Z>(pz.L, fft_generic, [&](auto lc) {
         if (o32)
             hipLaunchKernelGGL((k_zmi<T, decltype(lc)::value, true>), dim3(ntz, g.Py), dim3(3 * tz * pz.tline), shz, s,
                                S2, kern, plane, g.Hx, g.Hp, g.Hy2, g.Py, g.nz, pz.dev<T>(), tz, xcd_remap, mtz,
@@ -965,87 +967,90 @@ template <typename T> int ConvImpl<T>::batch_2d(B2Desc<T> &d, int threads, size_
 // system (tsys) and that system's workgroup; descriptor fields are read
 // through global-address-space pointer types (gfield) so that the accesses
 // through them are global, not flat, operations.
-template <typename T> __global__ void kb_xfwd(const BxDesc<T> *__restrict__ D, const int *__restrict__ tsys)
+template <typename T, int LC> __global__ void kb_xfwd(const BxDesc<T> *__restrict__ D, const int *__restrict__ tsys)
 {
     const int gi = block_tile(1);
     const BxDesc<T> &d = D[tsys[gi]];
     if (gfield(d.stop)[0]) return;
     const T *in = gfield(d.sel)[0] ? gfield(d.y1) : gfield(d.y0);
-    xfwd_body<T, T, 0>(in, d.in_cstride, gfield(d.S1), d.out_cstride, d.Hx, d.Hp, d.ny, d.nz, d.nrows, d.nx, d.p,
+    xfwd_body<T, T, LC>(in, d.in_cstride, gfield(d.S1), d.out_cstride, d.Hx, d.Hp, d.ny, d.nz, d.nrows, d.nx, d.p,
                        d.lpw, gi - d.tbase);
 }
 
-template <typename T, bool INV, bool O32>
+template <typename T, bool INV, int LC, bool O32>
 __global__ void kb_y(const ByDesc<T> *__restrict__ D, const int *__restrict__ tsys)
 {
     const int gi = block_tile(1);
     const ByDesc<T> &d = D[tsys[gi]];
     if (gfield(d.stop)[0]) return;
     if (INV)
-        yinv_body<T, 0, O32>(gfield(d.S2), gfield(d.S1), d.Hx, d.Hp, d.ny, d.nz, d.p, d.tk, gi - d.tbase, d.ntx,
+        yinv_body<T, LC, O32>(gfield(d.S2), gfield(d.S1), d.Hx, d.Hp, d.ny, d.nz, d.p, d.tk, gi - d.tbase, d.ntx,
                              d.mtx, d.mzl);
     else
-        yfwd_body<T, 0, O32>(gfield(d.S1), gfield(d.S2), d.Hx, d.Hp, d.ny, d.nz, d.p, d.tk, gi - d.tbase, d.ntx,
+        yfwd_body<T, LC, O32>(gfield(d.S1), gfield(d.S2), d.Hx, d.Hp, d.ny, d.nz, d.p, d.tk, gi - d.tbase, d.ntx,
                              d.mtx, d.mzl);
 }
 
-template <typename T, bool O32> __global__ void kb_zmi(const BzDesc<T> *__restrict__ D, const int *__restrict__ tsys)
+template <typename T, int LC, bool O32> __global__ void kb_zmi(const BzDesc<T> *__restrict__ D, const int *__restrict__ tsys)
 {
     const int gi = block_tile(1);
     const BzDesc<T> &d = D[tsys[gi]];
     if (gfield(d.stop)[0]) return;
-    zmi_body<T, 0, O32>(gfield(d.S2), gfield(d.K), d.plane, d.Hx, d.Hp, d.Hy2, d.Py, d.nz, d.p, d.tk, 1, gi - d.tbase,
+    zmi_body<T, LC, O32>(gfield(d.S2), gfield(d.K), d.plane, d.Hx, d.Hp, d.Hy2, d.Py, d.nz, d.p, d.tk, 1, gi - d.tbase,
                         d.ntx, d.mtx, d.zsb, d.pb);
 }
 
-template <typename T> __global__ void kb_ymi2d(const B2Desc<T> *__restrict__ D, const int *__restrict__ tsys)
+template <typename T, int LC> __global__ void kb_ymi2d(const B2Desc<T> *__restrict__ D, const int *__restrict__ tsys)
 {
     const int gi = block_tile(1);
     const B2Desc<T> &d = D[tsys[gi]];
     if (gfield(d.stop)[0]) return;
-    ymi2d_body<T, 0>(gfield(d.S1), gfield(d.K), d.plane, d.Hx, d.Hp, d.Hy2, d.ny, d.p, d.tk, gi - d.tbase);
+    ymi2d_body<T, LC>(gfield(d.S1), gfield(d.K), d.plane, d.Hx, d.Hp, d.Hy2, d.ny, d.p, d.tk, gi - d.tbase);
 }
 
+// f(compiled plans, 32-bit offsets) of the launch
+template <int ANY, typename F> static void batch_kind(const BatchPass &bp, F &&f)
+{
+    if (bp.o32) {
+        if (bp.compiled) f(std::integral_constant<int, ANY>(), std::true_type());
+        else f(std::integral_constant<int, 0>(), std::true_type());
+    } else {
+        if (bp.compiled) f(std::integral_constant<int, ANY>(), std::false_type());
+        else f(std::integral_constant<int, 0>(), std::false_type());
+    }
+}
 template <typename T> void mm_batch_xfwd(const BatchPass &bp, hipStream_t s)
 {
-    hipLaunchKernelGGL(kb_xfwd<T>, dim3(bp.ntiles), dim3(bp.threads), bp.lds, s, (const BxDesc<T> *)bp.desc,
-                       (const int *)bp.tsys);
+    batch_kind<MM_LC_ANY>(bp, [&](auto lc, auto) {
+        hipLaunchKernelGGL((kb_xfwd<T, decltype(lc)::value>), dim3(bp.ntiles), dim3(bp.threads), bp.lds, s,
+                           (const BxDesc<T> *)bp.desc, (const int *)bp.tsys);
+    });
     MM_HIP(hipGetLastError());
 }
-template <typename T> void mm_batch_yfwd(const BatchPass &bp, hipStream_t s)
+template <typename T, bool INV> static void batch_y_pass(const BatchPass &bp, hipStream_t s)
 {
-    if (bp.o32)
-        hipLaunchKernelGGL((kb_y<T, false, true>), dim3(bp.ntiles), dim3(bp.threads), bp.lds, s,
-                           (const ByDesc<T> *)bp.desc, (const int *)bp.tsys);
-    else
-        hipLaunchKernelGGL((kb_y<T, false, false>), dim3(bp.ntiles), dim3(bp.threads), bp.lds, s,
-                           (const ByDesc<T> *)bp.desc, (const int *)bp.tsys);
+    batch_kind<MM_LC_ANY>(bp, [&](auto lc, auto o32) {
+        hipLaunchKernelGGL((kb_y<T, INV, decltype(lc)::value, decltype(o32)::value>), dim3(bp.ntiles),
+                           dim3(bp.threads), bp.lds, s, (const ByDesc<T> *)bp.desc, (const int *)bp.tsys);
+    });
     MM_HIP(hipGetLastError());
 }
-template <typename T> void mm_batch_yinv(const BatchPass &bp, hipStream_t s)
-{
-    if (bp.o32)
-        hipLaunchKernelGGL((kb_y<T, true, true>), dim3(bp.ntiles), dim3(bp.threads), bp.lds, s,
-                           (const ByDesc<T> *)bp.desc, (const int *)bp.tsys);
-    else
-        hipLaunchKernelGGL((kb_y<T, true, false>), dim3(bp.ntiles), dim3(bp.threads), bp.lds, s,
-                           (const ByDesc<T> *)bp.desc, (const int *)bp.tsys);
-    MM_HIP(hipGetLastError());
-}
+template <typename T> void mm_batch_yfwd(const BatchPass &bp, hipStream_t s) { batch_y_pass<T, false>(bp, s); }
+template <typename T> void mm_batch_yinv(const BatchPass &bp, hipStream_t s) { batch_y_pass<T, true>(bp, s); }
 template <typename T> void mm_batch_zmi(const BatchPass &bp, hipStream_t s)
 {
-    if (bp.o32)
-        hipLaunchKernelGGL((kb_zmi<T, true>), dim3(bp.ntiles), dim3(bp.threads), bp.lds, s,
-                           (const BzDesc<T> *)bp.desc, (const int *)bp.tsys);
-    else
-        hipLaunchKernelGGL((kb_zmi<T, false>), dim3(bp.ntiles), dim3(bp.threads), bp.lds, s,
-                           (const BzDesc<T> *)bp.desc, (const int *)bp.tsys);
+    batch_kind<MM_LC_Z>(bp, [&](auto lc, auto o32) {
+        hipLaunchKernelGGL((kb_zmi<T, decltype(lc)::value, decltype(o32)::value>), dim3(bp.ntiles), dim3(bp.threads),
+                           bp.lds, s, (const BzDesc<T> *)bp.desc, (const int *)bp.tsys);
+    });
     MM_HIP(hipGetLastError());
 }
 template <typename T> void mm_batch_ymi2d(const BatchPass &bp, hipStream_t s)
 {
-    hipLaunchKernelGGL(kb_ymi2d<T>, dim3(bp.ntiles), dim3(bp.threads), bp.lds, s, (const B2Desc<T> *)bp.desc,
-                       (const int *)bp.tsys);
+    batch_kind<MM_LC_ANY>(bp, [&](auto lc, auto) {
+        hipLaunchKernelGGL((kb_ymi2d<T, decltype(lc)::value>), dim3(bp.ntiles), dim3(bp.threads), bp.lds, s,
+                           (const B2Desc<T> *)bp.desc, (const int *)bp.tsys);
+    });
     MM_HIP(hipGetLastError());
 }
 template struct ConvImpl<MM_CONV_T>;

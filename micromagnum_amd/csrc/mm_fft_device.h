@@ -14,6 +14,7 @@
 #include <hip/hip_runtime.h>
 
 #define MM_FFT_MAX_PASSES 8
+#define MM_FFT_EPT 8  // elements of a line per thread
 
 template <typename T> struct cvec;
 template <> struct cvec<float> { typedef float2 type; };
@@ -94,6 +95,7 @@ struct FftPlanDev {
     const void *tw;        // per-pass twiddles (ntw entries), precision T
     int ntw;
     int pow2;              // L is a power of two (all radices 8, 4, 2)
+    int id;                // compiled plan of this length (mm_plan_id), 0: none
 };
 
 // The kernels copy the plan's twiddle table into LDS next to their lines
@@ -175,7 +177,9 @@ template <typename T, bool INV> __device__ __forceinline__ void dft5(C2<T> *v)
     const C2<T> a0 = v[0];
     const C2<T> m1 = cmk<T>(a0.x + c1 * b1.x + c2 * b2.x, a0.y + c1 * b1.y + c2 * b2.y);
     const C2<T> m2 = cmk<T>(a0.x + c2 * b1.x + c1 * b2.x, a0.y + c2 * b1.y + c1 * b2.y);
-    const C2<T> n1 = cmk<T>(sg * (s1 * d1.x + s2 * d2.x), sg * (s1 * d1.y + s2 * d2.y)); // times i below
+    // which product of a sum is the fused one is spelled out: left to the
+    // compiler it differed between kernels of one length
+    const C2<T> n1 = cmk<T>(sg * fma(s2, d2.x, s1 * d1.x), sg * fma(s2, d2.y, s1 * d1.y)); // times i below
     const C2<T> n2 = cmk<T>(sg * (s2 * d1.x - s1 * d2.x), sg * (s2 * d1.y - s1 * d2.y));
     v[0] = cmk<T>(a0.x + b1.x + b2.x, a0.y + b1.y + b2.y);
     v[1] = cmk<T>(m1.x - n1.y, m1.y + n1.x);
@@ -270,8 +274,6 @@ __device__ __forceinline__ void lds_fft_ept(C2<T> *line, const FftPlanDev &p, co
     }
 }
 
-#define MM_FFT_EPT 8
-
 template <typename T, bool INV, int SK>
 __device__ __forceinline__ void lds_fft(C2<T> *line, const FftPlanDev &p, int t, bool active, const C2<T> *tw)
 {
@@ -292,12 +294,11 @@ struct LineMap {
     bool active;
 };
 
-template <int R, int EPT, typename T, bool INV, bool P2, bool LDIN, bool STOUT, int SK, bool PRE, typename LD,
+template <int R, int MB, typename T, bool INV, bool P2, bool LDIN, bool STOUT, int SK, bool PRE, typename LD,
           typename ST, typename PF>
 __device__ __forceinline__ void fft_pass_io(C2<T> *lineG, LineMap g, C2<T> *lineS, LineMap sm_, const C2<T> *tw,
                                             int L, int tline, int Ns, int lNs, int toff, LD &ld, ST &st, PF &pre)
 {
-    constexpr int MB = MaxB<R, EPT>::value;
     const int nb = L / R;
     C2<T> v[MB][R];
     // a pass that reads through ld or writes through st runs in the global
@@ -368,17 +369,17 @@ __device__ __forceinline__ void fft_pass_sel(int R, C2<T> *lineG, LineMap g, C2<
     constexpr bool I = LDIN && FIRST, O = STOUT && LAST;
     if (P2) {
         switch (R) {
-        case 8: fft_pass_io<8, EPT, T, INV, true, I, O, SK, FIRST>(lineG, g, lineS, s_, tw, L, tline, Ns, lNs, toff, ld, st, pre); break;
-        case 4: fft_pass_io<4, EPT, T, INV, true, I, O, SK, FIRST>(lineG, g, lineS, s_, tw, L, tline, Ns, lNs, toff, ld, st, pre); break;
-        default: fft_pass_io<2, EPT, T, INV, true, I, O, SK, FIRST>(lineG, g, lineS, s_, tw, L, tline, Ns, lNs, toff, ld, st, pre); break;
+        case 8: fft_pass_io<8, MaxB<8, EPT>::value, T, INV, true, I, O, SK, FIRST>(lineG, g, lineS, s_, tw, L, tline, Ns, lNs, toff, ld, st, pre); break;
+        case 4: fft_pass_io<4, MaxB<4, EPT>::value, T, INV, true, I, O, SK, FIRST>(lineG, g, lineS, s_, tw, L, tline, Ns, lNs, toff, ld, st, pre); break;
+        default: fft_pass_io<2, MaxB<2, EPT>::value, T, INV, true, I, O, SK, FIRST>(lineG, g, lineS, s_, tw, L, tline, Ns, lNs, toff, ld, st, pre); break;
         }
     } else {
         switch (R) {
-        case 8: fft_pass_io<8, EPT, T, INV, false, I, O, SK, FIRST>(lineG, g, lineS, s_, tw, L, tline, Ns, 0, toff, ld, st, pre); break;
-        case 5: fft_pass_io<5, EPT, T, INV, false, I, O, SK, FIRST>(lineG, g, lineS, s_, tw, L, tline, Ns, 0, toff, ld, st, pre); break;
-        case 4: fft_pass_io<4, EPT, T, INV, false, I, O, SK, FIRST>(lineG, g, lineS, s_, tw, L, tline, Ns, 0, toff, ld, st, pre); break;
-        case 3: fft_pass_io<3, EPT, T, INV, false, I, O, SK, FIRST>(lineG, g, lineS, s_, tw, L, tline, Ns, 0, toff, ld, st, pre); break;
-        default: fft_pass_io<2, EPT, T, INV, false, I, O, SK, FIRST>(lineG, g, lineS, s_, tw, L, tline, Ns, 0, toff, ld, st, pre); break;
+        case 8: fft_pass_io<8, MaxB<8, EPT>::value, T, INV, false, I, O, SK, FIRST>(lineG, g, lineS, s_, tw, L, tline, Ns, 0, toff, ld, st, pre); break;
+        case 5: fft_pass_io<5, MaxB<5, EPT>::value, T, INV, false, I, O, SK, FIRST>(lineG, g, lineS, s_, tw, L, tline, Ns, 0, toff, ld, st, pre); break;
+        case 4: fft_pass_io<4, MaxB<4, EPT>::value, T, INV, false, I, O, SK, FIRST>(lineG, g, lineS, s_, tw, L, tline, Ns, 0, toff, ld, st, pre); break;
+        case 3: fft_pass_io<3, MaxB<3, EPT>::value, T, INV, false, I, O, SK, FIRST>(lineG, g, lineS, s_, tw, L, tline, Ns, 0, toff, ld, st, pre); break;
+        default: fft_pass_io<2, MaxB<2, EPT>::value, T, INV, false, I, O, SK, FIRST>(lineG, g, lineS, s_, tw, L, tline, Ns, 0, toff, ld, st, pre); break;
         }
     }
 }
@@ -428,21 +429,103 @@ __device__ __forceinline__ void fft_line_p2(const FftPlanDev &p, const C2<T> *tw
     }
 }
 
-// ---- compile-time plans for power-of-two lengths ---------------------------
-// A kernel instantiated for a fixed power-of-two length LC runs the passes of
-// the runtime plan (radix-8 passes, then one radix-4 or radix-2 pass, as
-// FftPlanHost::build orders them) with every length, stride and pass count a
-// constant: the pass loop unrolls, the radix switch disappears and the index
-// arithmetic folds (shorter code, no divisions, fewer live registers).
-constexpr int mm_ilog2(int v) { return v <= 1 ? 0 : 1 + mm_ilog2(v >> 1); }
+// ---- compile-time plans ----------------------------------------------------
+// A transform compiled for a fixed length LC runs its passes with every
+// length, stride and pass count a constant: the pass loop unrolls, the radix
+// switch disappears and the index arithmetic folds (shorter code, no
+// divisions, fewer live registers).  The passes are the runtime plan's, with
+// the same twiddles and the same arithmetic per element, so both give the
+// same bits.  Powers of two have kernels of their own; the other even lengths
+// of the table (a mesh's padded size is one of them up to 500 points, and the
+// common ones up to 1000) run in one kernel per pass that selects the length
+// at its start (LC < 0).  Against the loop of the runtime plan, MI355X:
+// 150x90x14 FP32 (300, 180, 30 points) y passes 10.3 / 8.5 -> 8.0 / 7.4 us,
+// z 20.0 -> 16.9 us, stage 32 -> 17.8 us; 99x85x7 FP32 field 35.2 -> 25.8 us.
+// Two neighbouring passes run as one in registers (radix up to 16) were no
+// faster: the selecting kernel has the registers of its largest pass.
+#define MM_FFT_POW2(X) X(2) X(4) X(8) X(16) X(32) X(64) X(128) X(256) X(512) X(1024) X(2048)
+#define MM_FFT_MIXED_Z(X)                                                                                         \
+    X(6) X(10) X(12) X(18) X(20) X(24) X(30) X(36) X(40) X(48) X(50) X(54) X(60) X(72) X(80) X(90) X(96) X(100)   \
+    X(108) X(120)
+#define MM_FFT_MIXED_XY(X)                                                                                        \
+    X(144) X(150) X(160) X(162) X(180) X(192) X(200) X(216) X(240) X(250) X(270) X(288) X(300) X(320) X(324)      \
+    X(360) X(384) X(400) X(432) X(450) X(480) X(486) X(500) X(540) X(576) X(600) X(640) X(648) X(720) X(750)      \
+    X(768) X(800) X(900) X(960) X(1000)
+
+// number of a compiled length in the tables, 0 if it is in none
+constexpr int mm_plan_id(int L)
+{
+    int id = 0, found = 0;
+#define MM_FFT_X(N) ++id; if (L == N) found = id;
+    MM_FFT_POW2(MM_FFT_X) MM_FFT_MIXED_Z(MM_FFT_X) MM_FFT_MIXED_XY(MM_FFT_X)
+#undef MM_FFT_X
+    return found;
+}
+// the z pass has the length compiled
+constexpr bool mm_plan_z(int L)
+{
+    bool found = L <= 128 && L >= 2 && (L & (L - 1)) == 0;
+#define MM_FFT_X(N) found = found || L == N;
+    MM_FFT_MIXED_Z(MM_FFT_X)
+#undef MM_FFT_X
+    return found;
+}
+
+// passes of a length 2^a 3^b 5^c: radix 8 while it divides, then one 4 or 2,
+// then the fives, then the threes; n = 0 if there is another factor
+struct FftRadices {
+    int n, r[16];
+};
+constexpr FftRadices mm_plan_radices(int L)
+{
+    FftRadices f = {0, {}};
+    int m = L, twos = 0;
+    for (; m % 2 == 0; m /= 2) ++twos;
+    for (; twos >= 3; twos -= 3) f.r[f.n++] = 8;
+    if (twos) f.r[f.n++] = 1 << twos;
+    for (; m % 5 == 0; m /= 5) f.r[f.n++] = 5;
+    for (; m % 3 == 0; m /= 3) f.r[f.n++] = 3;
+    if (m != 1) f.n = 0;
+    return f;
+}
+// Threads per line of a compiled length.  Powers of two: L/8.  Else the count
+// that wastes the fewest thread slots over the passes (each deals its butterflies
+// out in rounds of that many), counting a butterfly's arithmetic and element
+// accesses, times a tenth more per round (the line's latency); equal counts
+// go to the wider one.  At least a twelfth of the
+// line, which the z pass's kernel items need.
+constexpr int mm_plan_tline(int L)
+{
+    if ((L & (L - 1)) == 0) return L > MM_FFT_EPT ? L / MM_FFT_EPT : 1;
+    const FftRadices f = mm_plan_radices(L);
+    int most = 1, best = 1;
+    long cost = -1;
+    for (int p = 0; p < f.n; ++p) most = L / f.r[p] > most ? L / f.r[p] : most;
+    for (int t = (L / 2 + 6) / 6; t <= most || cost < 0; ++t) {
+        long c = 0, rounds = 10;
+        for (int p = 0; p < f.n; ++p) {
+            const int R = f.r[p], nb = L / R, mb = (nb + t - 1) / t;
+            c += (long)mb * t * (R * R / 3 + 10 * R + 20);
+            rounds += mb;
+        }
+        c *= rounds;
+        if (cost < 0 || c <= cost) {
+            cost = c;
+            best = t;
+        }
+    }
+    return best;
+}
 
 template <int LC> struct FftLen {
-    static_assert(LC >= 2 && (LC & (LC - 1)) == 0, "compile-time plans are for powers of two");
-    static constexpr int lg = mm_ilog2(LC);
-    static constexpr int n8 = lg / 3, rem = lg % 3;
-    static constexpr int npass = n8 + (rem ? 1 : 0);
-    static constexpr int tline = LC > MM_FFT_EPT ? LC / MM_FFT_EPT : 1;
-    static constexpr int radix(int ps) { return ps < n8 ? 8 : (rem == 2 ? 4 : 2); }
+    static constexpr FftRadices f = mm_plan_radices(LC);
+    static_assert(f.n > 0 && LC > 1, "no compiled plan of this length");
+    static constexpr int npass = f.n;
+    static constexpr bool p2 = (LC & (LC - 1)) == 0;
+    static constexpr int tline = mm_plan_tline(LC);
+    static constexpr int radix(int ps) { return f.r[ps]; }
+    // butterflies per thread of pass ps
+    static constexpr int mb(int ps) { return (LC / f.r[ps] + tline - 1) / tline; }
     // offset of pass ps in the per-pass twiddle table
     static constexpr int toff(int ps)
     {
@@ -455,16 +538,24 @@ template <int LC> struct FftLen {
     }
 };
 
+constexpr int mm_ilog2(int v) { return v <= 1 ? 0 : 1 + mm_ilog2(v >> 1); }
+
 // line length and threads per line of a kernel instantiated for LC (0: the
-// runtime plan p)
+// runtime plan p; MM_LC_ANY, MM_LC_Z: a compiled length selected at run time,
+// any or one of the z pass's)
+#define MM_LC_ANY (-1)
+#define MM_LC_Z (-2)
 template <int LC> struct PlanC {
     __device__ static constexpr int L(const FftPlanDev &) { return LC; }
     __device__ static constexpr int tline(const FftPlanDev &) { return FftLen<LC>::tline; }
 };
-template <> struct PlanC<0> {
+struct PlanRun {
     __device__ static int L(const FftPlanDev &p) { return p.L; }
     __device__ static int tline(const FftPlanDev &p) { return p.tline; }
 };
+template <> struct PlanC<0> : PlanRun {};
+template <> struct PlanC<MM_LC_ANY> : PlanRun {};
+template <> struct PlanC<MM_LC_Z> : PlanRun {};
 
 template <typename T, bool INV, int LC, int PS, int NS, bool LDIN, bool STOUT, int SK, typename LD, typename ST,
           typename PF>
@@ -475,14 +566,14 @@ __device__ __forceinline__ void fft_line_c(const C2<T> *tw, C2<T> *lineG, LineMa
     if constexpr (PS < F::npass) {
         constexpr int R = F::radix(PS);
         constexpr bool I = LDIN && PS == 0, O = STOUT && PS == F::npass - 1;
-        fft_pass_io<R, MM_FFT_EPT, T, INV, true, I, O, SK, PS == 0>(lineG, g, lineS, s_, tw, LC, F::tline, NS,
+        fft_pass_io<R, F::mb(PS), T, INV, F::p2, I, O, SK, PS == 0>(lineG, g, lineS, s_, tw, LC, F::tline, NS,
                                                                     mm_ilog2(NS), F::toff(PS), ld, st, pre);
         fft_line_c<T, INV, LC, PS + 1, NS * R, LDIN, STOUT, SK>(tw, lineG, g, lineS, s_, ld, st, pre);
     }
 }
 
-// LC > 0: the compile-time plan of that length (p.L must equal LC); LC == 0:
-// the runtime plan p.  SK: the LDS skew of the lines (sk).
+// LC > 0: the compile-time plan of that length (p.L must equal LC); LC < 0:
+// the compiled length number p.id; LC == 0: the runtime plan p.  SK: the LDS skew of the lines (sk).
 struct FftNoPre {
     __device__ void operator()() const {}
 };
@@ -496,6 +587,24 @@ __device__ __forceinline__ void fft_line(const FftPlanDev &p, const C2<T> *tw, C
 {
     if constexpr (LC > 0) {
         fft_line_c<T, INV, LC, 0, 1, LDIN, STOUT, SK>(tw, lineG, g, lineS, s_, ld, st, pre);
+    } else if constexpr (LC < 0) {
+        // one workgroup runs one length: a uniform jump
+#define MM_FFT_X(N) case mm_plan_id(N): fft_line_c<T, INV, N, 0, 1, LDIN, STOUT, SK>(tw, lineG, g, lineS, s_, ld, st, pre); break;
+        if constexpr (LC == MM_LC_Z) {
+            switch (p.id) {
+            MM_FFT_X(2) MM_FFT_X(4) MM_FFT_X(8) MM_FFT_X(16) MM_FFT_X(32) MM_FFT_X(64) MM_FFT_X(128)
+            MM_FFT_MIXED_Z(MM_FFT_X)
+            default: break;
+            }
+        } else {
+            switch (p.id) {
+            MM_FFT_POW2(MM_FFT_X)
+            MM_FFT_MIXED_Z(MM_FFT_X)
+            MM_FFT_MIXED_XY(MM_FFT_X)
+            default: break;
+            }
+        }
+#undef MM_FFT_X
     } else {
         if (p.pow2) fft_line_p2<T, INV, true, LDIN, STOUT, SK>(p, tw, lineG, g, lineS, s_, ld, st, pre);
         else fft_line_p2<T, INV, false, LDIN, STOUT, SK>(p, tw, lineG, g, lineS, s_, ld, st, pre);

@@ -841,12 +841,12 @@ template <typename T> struct BStageDesc {
     FftPlanDev p;
 };
 
-template <typename T, bool STT, bool GEN, bool P1S = false>
+template <typename T, int LC, bool STT, bool GEN, bool P1S = false>
 __global__ void kb_stage(const BStageDesc<T> *__restrict__ D, const int *__restrict__ tsys, int st)
 {
     const int gi = block_tile(1);
     const BStageDesc<T> &d = D[tsys[gi]];
-    stage_body<T, false, 0, STT, GEN, P1S>(gfield(d.S), gfield(d.G0) + st, gfield(d.ctl), gfield(d.S1), d.p, d.Hx, d.Hp,
+    stage_body<T, false, LC, STT, GEN, P1S>(gfield(d.S), gfield(d.G0) + st, gfield(d.ctl), gfield(d.S1), d.p, d.Hx, d.Hp,
                                       d.rpw, 1, nullptr, nullptr, gi - d.tbase, d.nb, false);
 }
 

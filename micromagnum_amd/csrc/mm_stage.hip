@@ -30,8 +30,12 @@ template int stage_blocks_per_cu<MM_STAGE_T, MM_STAGE_STT, MM_STAGE_GEN>(int, bo
 
 template <typename T, bool STT, bool GEN, bool P1S> void stage_run_batch(const BatchPass &bp, hipStream_t s, int st)
 {
-    hipLaunchKernelGGL((kb_stage<T, STT, GEN, P1S>), dim3(bp.ntiles), dim3(bp.threads), bp.lds, s,
-                       (const BStageDesc<T> *)bp.desc, (const int *)bp.tsys, st);
+    if (bp.compiled)
+        hipLaunchKernelGGL((kb_stage<T, MM_LC_ANY, STT, GEN, P1S>), dim3(bp.ntiles), dim3(bp.threads), bp.lds, s,
+                           (const BStageDesc<T> *)bp.desc, (const int *)bp.tsys, st);
+    else
+        hipLaunchKernelGGL((kb_stage<T, 0, STT, GEN, P1S>), dim3(bp.ntiles), dim3(bp.threads), bp.lds, s,
+                           (const BStageDesc<T> *)bp.desc, (const int *)bp.tsys, st);
     MM_HIP(hipGetLastError());
 }
 template void stage_run_batch<MM_STAGE_T, MM_STAGE_STT, MM_STAGE_GEN, MM_STAGE_P1S>(const BatchPass &, hipStream_t, int);

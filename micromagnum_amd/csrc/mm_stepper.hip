@@ -576,11 +576,18 @@ template <typename T> struct Stepper : public StepperBase {
                     threads = t;
                 }
             }
-            // fewer workgroups than CUs: the launch takes as long as one
-            // workgroup, so every cell gets its own thread.  128x32x1 FP64:
-            // stage 16.1 -> 9.8 us with the one-pair workgroups above
-            if (!ext && (d.ny * d.nz + rpw - 1) / rpw <= num_cus())
-                threads = std::min(1024, std::max(fft_threads, rpw * ((d.nx + 63) / 64 * 64)));
+            // a launch whose workgroups are all resident at once takes as
+            // long as one of them: the most threads (up to one per cell) that
+            // keep it so.  128x32x1 FP64: stage 16.1 -> 9.8 us with the
+            // one-pair workgroups above; 150x90x14 FP32: 26.5 -> 17.8 us.
+            if (!ext) {
+                const int wgs = (d.ny * d.nz + rpw - 1) / rpw, cus = num_cus();
+                for (int t = std::min(1024, std::max(fft_threads, rpw * ((d.nx + 63) / 64 * 64))); t > threads; t -= 64)
+                    if (stage_occupancy(t) * cus >= wgs) {
+                        threads = t;
+                        break;
+                    }
+            }
             if (wshape.stage_threads > 0)
                 threads = std::min(1024, std::max(fft_threads, (wshape.stage_threads + 63) / 64 * 64));
             if (const char *e = std::getenv("MM_STAGE_THREADS"))
@@ -1736,6 +1743,13 @@ template <typename T> struct BatchRunner : BatchRunnerBase {
                 tz = std::max(tz, 3 * c.ln.tk_z * c.pz.tline);
             }
             tsg = std::max(tsg, q->threads);
+            bx.compiled = bx.compiled && c.px.id > 0;
+            if (c.g.is2d) {
+                b2.compiled = b2.compiled && c.py.id > 0;
+            } else {
+                by.compiled = by.compiled && c.py.id > 0;
+                bz.compiled = bz.compiled && mm_plan_z(c.pz.L);
+            }
         }
         bx.threads = round64(tx);
         by.threads = round64(ty);
@@ -1800,6 +1814,7 @@ template <typename T> struct BatchRunner : BatchRunnerBase {
             gr.stt = stt;
             gr.gen = gen;
             gr.bp.threads = round64(tsg);
+            gr.bp.compiled = bx.compiled;
             for (int i = 0; i < n; ++i) {
                 Stepper<T> *q = sys[i];
                 bool a, b;
