@@ -139,6 +139,26 @@ static inline unsigned mdiv(unsigned d, size_t nmax, bool wide = false)
     return (unsigned)((1ull << 32) / d + 1);
 }
 
+// n / d for the tile indices of a launch without an integer division (the
+// GPU has none; the compiler emits some twenty instructions for one):
+// m = floor(2^32 / d) + 1 gives floor(n / d) = umulhi(n, m) exactly when
+// n * d < 2^32.  mdiv returns 0 where that does not hold, and the division
+// is then done the long way.
+__device__ __forceinline__ unsigned udiv(unsigned n, unsigned d, unsigned m)
+{
+    return d == 1 ? n : (m ? __umulhi(n, m) : n / d);
+}
+
+// Fourier kernel times spectrum of one point; k: xx, xy, xz, yy, yz, zz
+template <typename T>
+__device__ __forceinline__ void mult3(C2<T> &mx, C2<T> &my, C2<T> &mz, const T k[6])
+{
+    const C2<T> x = mx, y = my, z = mz;
+    mx = cmk<T>(k[0] * x.x + k[1] * y.x + k[2] * z.x, k[0] * x.y + k[1] * y.y + k[2] * z.y);
+    my = cmk<T>(k[1] * x.x + k[3] * y.x + k[4] * z.x, k[1] * x.y + k[3] * y.y + k[4] * z.y);
+    mz = cmk<T>(k[2] * x.x + k[4] * y.x + k[5] * z.x, k[2] * x.y + k[4] * y.y + k[5] * z.y);
+}
+
 static inline int floor_pow2(int v) { return v < 1 ? 1 : 1 << (31 - __builtin_clz((unsigned)v)); }
 
 static inline int env_int(const char *name, int dflt)
@@ -286,11 +306,31 @@ struct ConvImpl {
     int batch_y(ByDesc<T> &d, int threads, size_t &lds, bool &o32, const int *stop) const;
     int batch_z(BzDesc<T> &d, int threads, size_t &lds, bool &o32, const int *stop) const;
     int batch_2d(B2Desc<T> &d, int threads, size_t &lds, const int *stop) const;
+    // The z pass takes its register form (mm_conv_zreg.hip).  Both forms on
+    // MI355X, field evaluation, LDS form -> register form: 200x200x5 (12
+    // points) FP32 49.6 -> 43.8 us, FP64 74.3 -> 60.0; 256x256x5 FP64 86.1 ->
+    // 66.0; 256x256x4 (8 points) FP32 41.0 -> 40.4, FP64 54.1 -> 53.4;
+    // 256x256x8 (16 points) FP32 58.9 -> 56.8, 99x85x8 28.3 -> 29.0: with
+    // less than a wave per SIMD the longer chain of one thread shows, and at
+    // 16 points it costs more than the barriers it saves.  FP64 lines of 16
+    // points leave one wave per SIMD (200x200x8: 83.9 -> 87.7), 20 and more
+    // likewise in FP32 (99x85x9: 29.7 -> 31.5, 256x256x16: 93.7 -> 105).
+    bool zreg() const
+    {
+        const int L = g.Pz;
+        const size_t cells = (size_t)g.Py * g.Hp;
+        const bool len = L == 4 || L == 6 || L == 8 || L == 10 || L == 12 ||
+                         (L == 16 && sizeof(T) == 4 && cells >= 65536);
+        return len && !g.is2d && !fft_generic && g.nz <= (L + 1) / 2 && cells * sizeof(C2<T>) < (1ull << 32);
+    }
     // threads per workgroup this system's passes need at least
     int batch_threads_x() const { return px.tline; }
     int batch_threads_y() const { return (g.is2d ? 3 : 1) * py.tline; }
     int batch_threads_z() const { return 3 * pz.tline; }
 };
+
+// z pass in registers (ConvImpl::zreg)
+template <typename T> void mm_zreg_pass(const ConvImpl<T> &c, hipStream_t s);
 
 // batched launches (all systems of bp in one launch on stream s)
 template <typename T> void mm_batch_xfwd(const BatchPass &bp, hipStream_t s);

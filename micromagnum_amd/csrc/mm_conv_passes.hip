@@ -91,16 +91,6 @@ __global__ void k_xfwd(const TIN *__restrict__ in, size_t in_cstride, C2<T> *__r
     xfwd_body<T, TIN, LC>(in, in_cstride, out, out_cstride, Hx, Hp, ny, nz, nrows, nx_in, p, lpw, (int)blockIdx.x);
 }
 
-// n / d for the tile indices of a launch without an integer division (the
-// GPU has none; the compiler emits some twenty instructions for one):
-// m = floor(2^32 / d) + 1 gives floor(n / d) = umulhi(n, m) exactly when
-// n * d < 2^32.  mdiv returns 0 where that does not hold, and the division
-// is then done the long way.
-__device__ __forceinline__ unsigned udiv(unsigned n, unsigned d, unsigned m)
-{
-    return d == 1 ? n : (m ? __umulhi(n, m) : n / d);
-}
-
 // y forward: columns kx of planes (c, z); rows y < ny_in read, Py written.
 // O32: both arrays under 4 GiB and a row under 16 MiB: 32-bit byte offsets
 // from the kernel-argument bases, rows stepped by 24-bit multiplies
@@ -319,15 +309,6 @@ __device__ __forceinline__ void kernel_at(const T *__restrict__ K, size_t plane,
     k[3] = K[3 * plane + o];
     k[4] = sy * sz * K[4 * plane + o];
     k[5] = K[5 * plane + o];
-}
-
-template <typename T>
-__device__ __forceinline__ void mult3(C2<T> &mx, C2<T> &my, C2<T> &mz, const T k[6])
-{
-    const C2<T> x = mx, y = my, z = mz;
-    mx = cmk<T>(k[0] * x.x + k[1] * y.x + k[2] * z.x, k[0] * x.y + k[1] * y.y + k[2] * z.y);
-    my = cmk<T>(k[1] * x.x + k[3] * y.x + k[4] * z.x, k[1] * x.y + k[3] * y.y + k[4] * z.y);
-    mz = cmk<T>(k[2] * x.x + k[4] * y.x + k[5] * z.x, k[2] * x.y + k[4] * y.y + k[5] * z.y);
 }
 
 // kernel items (column, kz pair) per thread of the z pass
@@ -805,7 +786,8 @@ template <typename T> void ConvImpl<T>::spectral(hipStream_t s)
     const size_t zsb = (size_t)g.Py * g.Hp * cs;
     const bool o32 = zsb < (1u << 24) && 3 * (size_t)g.nz * zsb < (1ull << 32) &&
                      kern_elems * sizeof(T) < (1ull << 32) && !wide;
-    mm_with_len<MM_LC_Z>(pz.L, fft_generic, [&](auto lc) {
+    if (zreg()) mm_zreg_pass<T>(*this, s);
+    else mm_with_len<MM_LC_Z>(pz.L, fft_generic, [&](auto lc) {
         if (o32)
             hipLaunchKernelGGL((k_zmi<T, decltype(lc)::value, true>), dim3(ntz, g.Py), dim3(3 * tz * pz.tline), shz, s,
                                S2, kern, plane, g.Hx, g.Hp, g.Hy2, g.Py, g.nz, pz.dev<T>(), tz, xcd_remap, mtz,
