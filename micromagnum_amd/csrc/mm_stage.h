@@ -58,6 +58,14 @@ template <typename T> struct VParam {
 
 enum { FORM_SUM = 0, FORM_SEQ = 1 };
 
+// Physics compiled into a stage kernel beyond uniform exchange, uniaxial
+// anisotropy and Zeeman field.  GEN_CUB: cubic anisotropy.  GEN_ALL: that,
+// exchange with per-cell Ms/A and 64-bit addresses.
+// Cubic anisotropy ran in GEN_ALL before, whose FP32 inner stage spilled
+// registers at 8 waves per SIMD: 512x512x32 FP32 inner stages 344 -> 300 us,
+// final 392 -> 374 us, 1 ps 124 -> 116 ms.
+enum StageGen { GEN_NONE = 0, GEN_ALL = 1, GEN_CUB = 2 };
+
 template <typename T> struct SysDev {
     MeshDev m;
     size_t n;
@@ -322,17 +330,18 @@ struct EnergyAcc {
 };
 
 // Per-cell epilogue: everything after the demag field of one cell.  STT:
-// the Zhang-Li term is compiled in; GEN: cubic anisotropy and the exchange
-// with per-cell Ms/A are compiled in (without them the epilogue is shorter
-// and needs fewer registers).  Without GEN the state arrays are addressed by
-// 32-bit byte offsets from their (workgroup-uniform) bases, which the host
-// guarantees by taking GEN for state arrays of 4 GiB or more.
-template <typename T, bool EN, bool STT, bool GEN, bool P1S = false>
+// the Zhang-Li term is compiled in; GEN (StageGen): which of cubic anisotropy
+// and the exchange with per-cell Ms/A are compiled in (without them the
+// epilogue is shorter and needs fewer registers).  Except in GEN_ALL the state
+// arrays are addressed by 32-bit byte offsets from their (workgroup-uniform)
+// bases, which the host guarantees by taking GEN_ALL for state arrays of
+// 4 GiB or more.
+template <typename T, bool EN, bool STT, int GEN, bool P1S = false>
 __device__ __forceinline__ void stage_cell(const SysDev<T> &S, const StageDev<T> &G, const StepCtl *ctl,
                                            const T *__restrict__ Y, int x, int y, int z, const V3<T> &Hd,
                                            const V3<T> &hz, StageRed &red, EnergyAcc &ea, T *nxt)
 {
-    constexpr bool O32 = !GEN;
+    constexpr bool O32 = GEN != GEN_ALL, CUB = GEN != GEN_NONE;
     const size_t n = S.n;
     const size_t i = (size_t)x + (size_t)S.m.nx * ((size_t)y + (size_t)S.m.ny * z);
     // byte offsets of cell i and of one component plane (O32 only)
@@ -376,15 +385,24 @@ __device__ __forceinline__ void stage_cell(const SysDev<T> &S, const StageDev<T>
                      : exchange_cell_inv<T>(S.m, x, y, z, i, n, S.wx, S.wy, S.wz, S.coef_ex,
                                         [&](long j) { return gfield(S.iMs)[j]; }, gfield(S.A.p), Y);
         }
-        H.x += he.x;
-        H.y += he.y;
-        H.z += he.z;
+        if constexpr (GEN == GEN_CUB) {
+            // rounded before the sum, as GEN_ALL has it (there the field comes
+            // from one of two branches): the same bits in both classes
+#pragma clang fp contract(off)
+            H.x += he.x;
+            H.y += he.y;
+            H.z += he.z;
+        } else {
+            H.x += he.x;
+            H.y += he.y;
+            H.z += he.z;
+        }
         if (EN) dd_add(ea.exch, dotd<T>(Mv, he));
     }
-    if (has_uni || (GEN && S.has_cub)) {
+    if (has_uni || (CUB && S.has_cub)) {
         T e0 = (T)0, e1 = (T)0;
         V3<T> ha = v3<T>(0, 0, 0);
-        if (GEN && S.has_cub) ha = cubic_cell<T>(Mv, S.axis1.at(n, i), S.axis2.at(n, i), S.kcub.at(i), ms, S.cm2mu0, &e1);
+        if (CUB && S.has_cub) ha = cubic_cell<T>(Mv, S.axis1.at(n, i), S.axis2.at(n, i), S.kcub.at(i), ms, S.cm2mu0, &e1);
         if (has_uni) {
             V3<T> hu;
             if (uni_fast) {
@@ -399,7 +417,7 @@ __device__ __forceinline__ void stage_cell(const SysDev<T> &S, const StageDev<T>
                 hu = uniaxial_cell<T>(Mv, S.axis1.at(n, i), S.kuni.at(i), ms, S.mu0, &e0);
             }
             if (EN) dd_add(ea.aniso, (double)e0);
-            if (GEN && S.has_cub) {
+            if (CUB && S.has_cub) {
                 ha.x += hu.x;
                 ha.y += hu.y;
                 ha.z += hu.z;
@@ -407,7 +425,7 @@ __device__ __forceinline__ void stage_cell(const SysDev<T> &S, const StageDev<T>
                 ha = hu;
             }
         }
-        if (EN && GEN && S.has_cub) dd_add(ea.aniso, (double)e1);
+        if (EN && CUB && S.has_cub) dd_add(ea.aniso, (double)e1);
         H.x += ha.x;
         H.y += ha.y;
         H.z += ha.z;
@@ -591,7 +609,7 @@ __device__ __forceinline__ void stage_cell(const SysDev<T> &S, const StageDev<T>
 // workgroup's index among the nblk of the system's launch; remap: order the
 // tiles by xcd_tile(blk, nblk) (the single-system launch; a batched launch
 // orders its global workgroups before it picks the system).
-template <typename T, bool EN, int LC, bool STT, bool GEN, bool P1S = false>
+template <typename T, bool EN, int LC, bool STT, int GEN, bool P1S = false>
 __device__ __forceinline__ void stage_body(const SysDev<T> *__restrict__ Sp, const StageDev<T> *__restrict__ Gp,
                                            StepCtl *ctl, const C2<T> *__restrict__ S1, const FftPlanDev &p, int Hx,
                                            int Hp, int rpw, int has_demag, double *__restrict__ epart,
@@ -820,7 +838,7 @@ __device__ __forceinline__ void stage_body(const SysDev<T> *__restrict__ Sp, con
 // SGPRs; asking for 8 (SGPRs 78, the rest spilled to VGPR lanes, no
 // scratch) lets a CU hold 8 of its 256-thread workgroups, one round for
 // 256x256x16 cells: stage 32.4 -> 30.7 us (MI355X, same-run A/B).
-template <typename T, bool EN, int LC, bool STT, bool GEN, bool P1S = false>
+template <typename T, bool EN, int LC, bool STT, int GEN, bool P1S = false>
 __global__ void __attribute__((amdgpu_waves_per_eu((P1S && sizeof(T) == 4) ? 8 : 1))) k_stage(const SysDev<T> *__restrict__ Sp, const StageDev<T> *__restrict__ Gp, StepCtl *ctl,
                         const C2<T> *__restrict__ S1, FftPlanDev p, int Hx, int Hp, int rpw, int has_demag,
                         double *__restrict__ epart, const T *__restrict__ Hdem)
@@ -841,7 +859,7 @@ template <typename T> struct BStageDesc {
     FftPlanDev p;
 };
 
-template <typename T, int LC, bool STT, bool GEN, bool P1S = false>
+template <typename T, int LC, bool STT, int GEN, bool P1S = false>
 __global__ void kb_stage(const BStageDesc<T> *__restrict__ D, const int *__restrict__ tsys, int st)
 {
     const int gi = block_tile(1);
@@ -870,12 +888,11 @@ template <typename T> struct StageArgs {
     const T *Hdem;
 };
 // the kernel of a physics class: EN the energy sums, STT Zhang-Li torque, GEN
-// cubic anisotropy or per-cell exchange, P1S inner stages with a summed
-// combination
-template <typename T, bool EN, bool STT, bool GEN, bool P1S> void stage_run(const StageArgs<T> &a);
+// the StageGen class, P1S inner stages with a summed combination
+template <typename T, bool EN, bool STT, int GEN, bool P1S> void stage_run(const StageArgs<T> &a);
 // workgroups of the (non-energy) kernel that one CU holds
-template <typename T, bool STT, bool GEN> int stage_blocks_per_cu(int len, bool generic, int threads, size_t lds);
+template <typename T, bool STT, int GEN> int stage_blocks_per_cu(int len, bool generic, int threads, size_t lds);
 // stage st of every system of a batch
-template <typename T, bool STT, bool GEN, bool P1S> void stage_run_batch(const BatchPass &bp, hipStream_t s, int st);
+template <typename T, bool STT, int GEN, bool P1S> void stage_run_batch(const BatchPass &bp, hipStream_t s, int st);
 
 #endif

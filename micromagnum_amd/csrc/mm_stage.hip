@@ -3,7 +3,7 @@
 // MM_STAGE_GEN, MM_STAGE_P1S); the Makefile builds one object per class.
 #include "mm_stage.h"
 
-template <typename T, bool EN, bool STT, bool GEN, bool P1S> void stage_run(const StageArgs<T> &a)
+template <typename T, bool EN, bool STT, int GEN, bool P1S> void stage_run(const StageArgs<T> &a)
 {
     mm_with_len(a.len, a.generic, [&](auto lc) {
         hipLaunchKernelGGL((k_stage<T, EN, decltype(lc)::value, STT, GEN, P1S>), dim3(a.grid), dim3(a.threads), a.lds,
@@ -16,7 +16,7 @@ template void stage_run<MM_STAGE_T, MM_STAGE_EN, MM_STAGE_STT, MM_STAGE_GEN, MM_
 
 #if !MM_STAGE_EN
 #if !MM_STAGE_P1S
-template <typename T, bool STT, bool GEN> int stage_blocks_per_cu(int len, bool generic, int threads, size_t lds)
+template <typename T, bool STT, int GEN> int stage_blocks_per_cu(int len, bool generic, int threads, size_t lds)
 {
     int nb = 0;
     mm_with_len(len, generic, [&](auto lc) {
@@ -28,7 +28,7 @@ template <typename T, bool STT, bool GEN> int stage_blocks_per_cu(int len, bool 
 template int stage_blocks_per_cu<MM_STAGE_T, MM_STAGE_STT, MM_STAGE_GEN>(int, bool, int, size_t);
 #endif
 
-template <typename T, bool STT, bool GEN, bool P1S> void stage_run_batch(const BatchPass &bp, hipStream_t s, int st)
+template <typename T, bool STT, int GEN, bool P1S> void stage_run_batch(const BatchPass &bp, hipStream_t s, int st)
 {
     if (bp.compiled)
         hipLaunchKernelGGL((kb_stage<T, MM_LC_ANY, STT, GEN, P1S>), dim3(bp.ntiles), dim3(bp.threads), bp.lds, s,

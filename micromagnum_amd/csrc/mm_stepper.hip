@@ -686,14 +686,21 @@ template <typename T> struct Stepper : public StepperBase {
     int stage_len() const { return demag_mode() == 1 ? conv->px.L : 0; }
 
     // Gd: the stage record in device memory (gtab)
-    // the stage kernel's physics class: STT (Zhang-Li) and GEN (cubic
-    // anisotropy, exchange with per-cell Ms/A, or state arrays of 4 GiB or
-    // more, which the other instantiation addresses by 32-bit byte offsets)
-    void physics_class(bool &stt, bool &gen) const
+    // the stage kernel's physics class: STT (Zhang-Li) and the StageGen class.
+    // State arrays of 4 GiB or more take GEN_ALL, whose addresses are 64 bits.
+    void physics_class(bool &stt, int &gen) const
     {
         const bool big = 3.0 * (double)n * sizeof(T) >= 4294967296.0;
         stt = sys.has_stt != 0;
-        gen = sys.has_cub || (sys.has_exch && !sys.exch_uniform) || big;
+        gen = big || (sys.has_exch && !sys.exch_uniform) ? GEN_ALL : (sys.has_cub ? GEN_CUB : GEN_NONE);
+    }
+
+    // f(std::integral_constant) of a StageGen value
+    template <typename F> static auto with_gen(int gen, F &&f)
+    {
+        if (gen == GEN_ALL) return f(std::integral_constant<int, GEN_ALL>());
+        if (gen == GEN_CUB) return f(std::integral_constant<int, GEN_CUB>());
+        return f(std::integral_constant<int, GEN_NONE>());
     }
 
     static int num_cus()
@@ -708,14 +715,15 @@ template <typename T> struct Stepper : public StepperBase {
     // CU holds at thr threads, with the stage's dynamic LDS
     int stage_occupancy(int thr)
     {
-        bool stt, gen;
+        bool stt;
+        int gen;
         physics_class(stt, gen);
         const int L = stage_len();
         const bool g = conv && conv->fft_generic;
-        if (stt) return gen ? stage_blocks_per_cu<T, true, true>(L, g, thr, stage_lds)
-                            : stage_blocks_per_cu<T, true, false>(L, g, thr, stage_lds);
-        return gen ? stage_blocks_per_cu<T, false, true>(L, g, thr, stage_lds)
-                   : stage_blocks_per_cu<T, false, false>(L, g, thr, stage_lds);
+        return with_gen(gen, [&](auto c) {
+            return stt ? stage_blocks_per_cu<T, true, decltype(c)::value>(L, g, thr, stage_lds)
+                       : stage_blocks_per_cu<T, false, decltype(c)::value>(L, g, thr, stage_lds);
+        });
     }
 
     // The stage kernel of the physics present; the energy launch (EN) has no
@@ -723,7 +731,8 @@ template <typename T> struct Stepper : public StepperBase {
     // combination (the classes without spin torque have a kernel for it).
     template <bool EN> void stage_kernel(const StageDev<T> *Gd, double *ep, bool p1s = false)
     {
-        bool stt, gen;
+        bool stt;
+        int gen;
         physics_class(stt, gen);
         StageArgs<T> a;
         a.grid = grid_rows;
@@ -743,15 +752,13 @@ template <typename T> struct Stepper : public StepperBase {
         a.generic = conv && conv->fft_generic;
         a.epart = ep;
         a.Hdem = Hdem;
-        if constexpr (EN) {
-            gen ? stage_run<T, true, false, true, false>(a) : stage_run<T, true, false, false, false>(a);
-        } else if (stt) {
-            gen ? stage_run<T, false, true, true, false>(a) : stage_run<T, false, true, false, false>(a);
-        } else if (p1s) {
-            gen ? stage_run<T, false, false, true, true>(a) : stage_run<T, false, false, false, true>(a);
-        } else {
-            gen ? stage_run<T, false, false, true, false>(a) : stage_run<T, false, false, false, false>(a);
-        }
+        with_gen(gen, [&](auto c) {
+            constexpr int GEN = decltype(c)::value;
+            if constexpr (EN) stage_run<T, true, false, GEN, false>(a);
+            else if (stt) stage_run<T, false, true, GEN, false>(a);
+            else if (p1s) stage_run<T, false, false, GEN, true>(a);
+            else stage_run<T, false, false, GEN, false>(a);
+        });
     }
 
     // need_fwd: S1 does not yet hold the x transform of the stage input
@@ -1690,7 +1697,8 @@ template <typename T> struct BatchRunner : BatchRunnerBase {
     BatchPass bx, by, bz, b2;
     struct StageGroup {
         BatchPass bp;
-        bool stt, gen;
+        bool stt;
+        int gen;  // StageGen
     };
     std::vector<StageGroup> stg;
     BCtlDesc *cdesc = nullptr;
@@ -1806,8 +1814,9 @@ template <typename T> struct BatchRunner : BatchRunnerBase {
         }
         if (any2d) upload_pass(b2, d2, t2_s);
         // stage launches, one per physics class present
-        for (int cls = 0; cls < 4; ++cls) {
-            const bool stt = cls & 1, gen = (cls >> 1) & 1;
+        for (int cls = 0; cls < 6; ++cls) {
+            const bool stt = cls & 1;
+            const int gen = cls >> 1;
             std::vector<BStageDesc<T>> ds;
             std::vector<int> ts;
             StageGroup gr;
@@ -1817,7 +1826,8 @@ template <typename T> struct BatchRunner : BatchRunnerBase {
             gr.bp.compiled = bx.compiled;
             for (int i = 0; i < n; ++i) {
                 Stepper<T> *q = sys[i];
-                bool a, b;
+                bool a;
+                int b;
                 q->physics_class(a, b);
                 if (a != stt || b != gen) continue;
                 BStageDesc<T> e;
@@ -1879,15 +1889,12 @@ template <typename T> struct BatchRunner : BatchRunnerBase {
         // inner stages of a six-stage tableau (summed combination, no FSAL in
         // a batch): the kernel compiled for them
         const bool p1s = ns == 6 && st < ns - 1;
-        if (gr.stt) {
-            gr.gen ? stage_run_batch<T, true, true, false>(gr.bp, s, st)
-                   : stage_run_batch<T, true, false, false>(gr.bp, s, st);
-        } else if (gr.gen) {
-            stage_run_batch<T, false, true, false>(gr.bp, s, st);
-        } else {
-            p1s ? stage_run_batch<T, false, false, true>(gr.bp, s, st)
-                : stage_run_batch<T, false, false, false>(gr.bp, s, st);
-        }
+        Stepper<T>::with_gen(gr.gen, [&](auto c) {
+            constexpr int GEN = decltype(c)::value;
+            if (gr.stt) stage_run_batch<T, true, GEN, false>(gr.bp, s, st);
+            else if (GEN != GEN_ALL && p1s) stage_run_batch<T, false, GEN, GEN != GEN_ALL>(gr.bp, s, st);
+            else stage_run_batch<T, false, GEN, false>(gr.bp, s, st);
+        });
     }
 
     // one attempt of every system (the records of stage st < ns - 1 also
