@@ -323,6 +323,9 @@ struct ConvImpl {
                          (L == 16 && sizeof(T) == 4 && cells >= 65536);
         return len && !g.is2d && !fft_generic && g.nz <= (L + 1) / 2 && cells * sizeof(C2<T>) < (1ull << 32);
     }
+    // ... and of a batched launch, whose kernel holds the lines of one pass
+    // (4 and 8 points, 2 to 4 layers), for which both forms give the same bits
+    bool zreg_batch() const { return zreg() && (g.Pz == 4 || g.Pz == 8); }
     // threads per workgroup this system's passes need at least
     int batch_threads_x() const { return px.tline; }
     int batch_threads_y() const { return (g.is2d ? 3 : 1) * py.tline; }
@@ -331,6 +334,11 @@ struct ConvImpl {
 
 // z pass in registers (ConvImpl::zreg)
 template <typename T> void mm_zreg_pass(const ConvImpl<T> &c, hipStream_t s);
+// a system's descriptor and workgroup count in the batched form (zreg_batch),
+// and the launch of all of them
+#define MM_ZREG_BATCH_THREADS 256
+template <typename T> int mm_zreg_desc(const ConvImpl<T> &c, BzDesc<T> &d, const int *stop);
+template <typename T> void mm_batch_zreg(const BatchPass &bp, hipStream_t s);
 
 // batched launches (all systems of bp in one launch on stream s)
 template <typename T> void mm_batch_xfwd(const BatchPass &bp, hipStream_t s);

@@ -12,6 +12,91 @@
 #include "mm_conv.h"
 #include "mm_cell.h"
 
+// Size-R DFTs with every rounding spelled out as the LDS form's compiled code
+// has it, so that both forms give the same bits: a product that enters a sum
+// and a difference is fused into both, except in the last pass of the inverse
+// (SPLIT), where the LDS form's sums sit in the blocks of its guarded stores
+// and the product is rounded first.
+template <typename T, bool SPLIT> __device__ __forceinline__ void addsub(T e, T c, T x, T &sum, T &dif)
+{
+    if constexpr (SPLIT) {
+#pragma clang fp contract(off)
+        const T p = c * x;
+        sum = e + p;
+        dif = e - p;
+    } else {
+        sum = fma(c, x, e);
+        dif = fma(-c, x, e);
+    }
+}
+
+template <typename T, bool INV, bool SPLIT> __device__ __forceinline__ void dft3_reg(C2<T> *v)
+{
+    const T c = (T)-0.5;
+    const T s = INV ? (T)0.86602540378443864676372317075293618347140262690519
+                    : (T)-0.86602540378443864676372317075293618347140262690519;
+    const C2<T> t = cadd<T>(v[1], v[2]), d = csub<T>(v[1], v[2]);
+    const C2<T> m = cmk<T>(fma(c, t.x, v[0].x), fma(c, t.y, v[0].y));
+    v[0] = cadd<T>(v[0], t);
+    addsub<T, SPLIT>(m.x, -s, d.y, v[1].x, v[2].x);
+    addsub<T, SPLIT>(m.y, s, d.x, v[1].y, v[2].y);
+}
+
+template <typename T, bool INV, bool SPLIT> __device__ __forceinline__ void dft8_reg(C2<T> *v)
+{
+    C2<T> e[4] = {v[0], v[2], v[4], v[6]};
+    C2<T> o[4] = {v[1], v[3], v[5], v[7]};
+    dft4<T, INV>(e);
+    dft4<T, INV>(o);
+    const T h = (T)0.70710678118654752440084436210484903928483593768847;
+    const C2<T> o2 = cmul_mi<T, INV>(o[2]);
+    v[0] = cadd<T>(e[0], o[0]);
+    v[4] = csub<T>(e[0], o[0]);
+    addsub<T, SPLIT>(e[1].x, h, INV ? o[1].x - o[1].y : o[1].x + o[1].y, v[1].x, v[5].x);
+    addsub<T, SPLIT>(e[1].y, h, INV ? o[1].x + o[1].y : o[1].y - o[1].x, v[1].y, v[5].y);
+    v[2] = cadd<T>(e[2], o2);
+    v[6] = csub<T>(e[2], o2);
+    addsub<T, SPLIT>(e[3].x, INV ? -h : h, INV ? o[3].x + o[3].y : o[3].y - o[3].x, v[3].x, v[7].x);
+    addsub<T, SPLIT>(e[3].y, INV ? h : -h, INV ? o[3].x - o[3].y : o[3].x + o[3].y, v[3].y, v[7].y);
+}
+
+// The transform of a line in one thread's registers: the passes and twiddles
+// of fft_line, no LDS, no barriers.  tw is the plan's per-pass table in global
+// memory; its indices are constants and its base is uniform, so the twiddles
+// come in by scalar loads.
+template <typename T, bool INV, int LC, int PS = 0, int NS = 1>
+__device__ __forceinline__ void fft_reg(C2<T> (&v)[LC], const C2<T> *__restrict__ tw)
+{
+    using F = FftLen<LC>;
+    if constexpr (PS < F::npass) {
+        constexpr int R = F::radix(PS), nb = LC / R;
+        constexpr bool SPLIT = INV && PS == F::npass - 1;
+        C2<T> o[LC];
+#pragma unroll
+        for (int b = 0; b < nb; ++b) {
+            const int k = b % NS;
+            C2<T> u[R];
+#pragma unroll
+            for (int r = 0; r < R; ++r) {
+                u[r] = v[b + r * nb];
+                if (r > 0 && k > 0) {
+                    C2<T> w = tw[F::toff(PS) + (r - 1) * NS + k];
+                    if (INV) w.y = -w.y;
+                    u[r] = cmul<T>(u[r], w);
+                }
+            }
+            if constexpr (R == 8) dft8_reg<T, INV, SPLIT>(u);
+            else if constexpr (R == 3) dft3_reg<T, INV, SPLIT>(u);
+            else dftR<R, T, INV>(u);
+#pragma unroll
+            for (int r = 0; r < R; ++r) o[(b / NS) * NS * R + k + r * NS] = u[r];
+        }
+#pragma unroll
+        for (int j = 0; j < LC; ++j) v[j] = o[j];
+        fft_reg<T, INV, LC, PS + 1, NS * R>(v, tw);
+    }
+}
+
 // One thread holds the z lines of the three components of one (kx, ky).  Threads run over the rows' whole pitch, so a
 // wave's accesses are contiguous; (c, z) planes and kernel planes have uniform
 // bases and the thread's offset in a plane is one 32-bit value.  Needs
@@ -109,3 +194,49 @@ template <typename T> void mm_zreg_pass(const ConvImpl<T> &c, hipStream_t s)
     MM_HIP(hipGetLastError());
 }
 template void mm_zreg_pass<MM_CONV_T>(const ConvImpl<MM_CONV_T> &, hipStream_t);
+
+// Batched form: systems of one-pass lines, which need no twiddles.  A wider
+// choice of lengths would give every system the registers of the longest.
+template <typename T>
+__global__ __launch_bounds__(MM_ZREG_BATCH_THREADS) void kb_zmir(const BzDesc<T> *__restrict__ D,
+                                                                 const int *__restrict__ tsys)
+{
+    const int gi = block_tile(1);
+    const BzDesc<T> &d = D[tsys[gi]];
+    if (gfield(d.stop)[0]) return;
+    const unsigned cell = (unsigned)(gi - d.tbase) * blockDim.x + threadIdx.x;
+    if (d.p.L == 4)
+        zmir_body<T, 4>(gfield(d.S2), gfield(d.K), d.plane, d.Hx, d.Hp, d.Hy2, d.Py, d.nz, nullptr, 1, cell, d.mtx);
+    else if (d.p.L == 8)
+        zmir_body<T, 8>(gfield(d.S2), gfield(d.K), d.plane, d.Hx, d.Hp, d.Hy2, d.Py, d.nz, nullptr, 1, cell, d.mtx);
+}
+
+template <typename T> int mm_zreg_desc(const ConvImpl<T> &c, BzDesc<T> &d, const int *stop)
+{
+    const ConvGeom &g = c.g;
+    MM_REQUIRE(c.zreg_batch(), "system has no batched register form of the z pass");
+    const size_t cells = (size_t)g.Py * g.Hp;
+    const int nb = (int)((cells + MM_ZREG_BATCH_THREADS - 1) / MM_ZREG_BATCH_THREADS);
+    d = BzDesc<T>();
+    d.S2 = c.S2;
+    d.K = c.kern;
+    d.plane = (size_t)g.Hp * g.Hy2 * g.Hz2;
+    d.stop = stop;
+    d.Hx = g.Hx;
+    d.Hp = g.Hp;
+    d.Hy2 = g.Hy2;
+    d.Py = g.Py;
+    d.nz = g.nz;
+    d.mtx = mdiv((unsigned)g.Hp, (size_t)nb * MM_ZREG_BATCH_THREADS, c.wide);
+    d.p = c.pz.template dev<T>();
+    return nb;
+}
+
+template <typename T> void mm_batch_zreg(const BatchPass &bp, hipStream_t s)
+{
+    hipLaunchKernelGGL((kb_zmir<T>), dim3(bp.ntiles), dim3(bp.threads), 0, s, (const BzDesc<T> *)bp.desc,
+                       (const int *)bp.tsys);
+    MM_HIP(hipGetLastError());
+}
+template int mm_zreg_desc<MM_CONV_T>(const ConvImpl<MM_CONV_T> &, BzDesc<MM_CONV_T> &, const int *);
+template void mm_batch_zreg<MM_CONV_T>(const BatchPass &, hipStream_t);

@@ -611,39 +611,6 @@ __device__ __forceinline__ void fft_line(const FftPlanDev &p, const C2<T> *tw, C
     }
 }
 
-// The same transform with the whole line in one thread's registers: no LDS, no
-// barriers.  tw is the plan's per-pass table in global memory; its indices are
-// constants and its base is uniform, so the twiddles come in by scalar loads.
-template <typename T, bool INV, int LC, int PS = 0, int NS = 1>
-__device__ __forceinline__ void fft_reg(C2<T> (&v)[LC], const C2<T> *__restrict__ tw)
-{
-    using F = FftLen<LC>;
-    if constexpr (PS < F::npass) {
-        constexpr int R = F::radix(PS), nb = LC / R;
-        C2<T> o[LC];
-#pragma unroll
-        for (int b = 0; b < nb; ++b) {
-            const int k = b % NS;
-            C2<T> u[R];
-#pragma unroll
-            for (int r = 0; r < R; ++r) {
-                u[r] = v[b + r * nb];
-                if (r > 0 && k > 0) {
-                    C2<T> w = tw[F::toff(PS) + (r - 1) * NS + k];
-                    if (INV) w.y = -w.y;
-                    u[r] = cmul<T>(u[r], w);
-                }
-            }
-            dftR<R, T, INV>(u);
-#pragma unroll
-            for (int r = 0; r < R; ++r) o[(b / NS) * NS * R + k + r * NS] = u[r];
-        }
-#pragma unroll
-        for (int j = 0; j < LC; ++j) v[j] = o[j];
-        fft_reg<T, INV, LC, PS + 1, NS * R>(v, tw);
-    }
-}
-
 // Twiddles fetched into registers at kernel start and stored to LDS by the
 // first FFT pass's pre() hook, so the first pass's data reads do not wait for
 // the twiddle read: TwFetch<T>::fetch(p) / .store(twl).

@@ -1825,7 +1825,7 @@ template <typename T> struct BatchRunner : BatchRunnerBase {
     hipStream_t s = nullptr;
     int ns = 0;
     bool any3d = false, any2d = false;
-    BatchPass bx, by, bz, b2;
+    BatchPass bx, by, bz, bzr, b2;  // bzr: z lines in registers
     struct StageGroup {
         BatchPass bp;
         bool stt;
@@ -1879,7 +1879,7 @@ template <typename T> struct BatchRunner : BatchRunnerBase {
             } else {
                 any3d = true;
                 ty = std::max(ty, c.ln.tk_y * c.py.tline);
-                tz = std::max(tz, 3 * c.ln.tk_z * c.pz.tline);
+                if (!c.zreg_batch()) tz = std::max(tz, 3 * c.ln.tk_z * c.pz.tline);
             }
             tsg = std::max(tsg, q->threads);
             bx.compiled = bx.compiled && c.px.id > 0;
@@ -1887,7 +1887,7 @@ template <typename T> struct BatchRunner : BatchRunnerBase {
                 b2.compiled = b2.compiled && c.py.id > 0;
             } else {
                 by.compiled = by.compiled && c.py.id > 0;
-                bz.compiled = bz.compiled && mm_plan_z(c.pz.L);
+                if (!c.zreg_batch()) bz.compiled = bz.compiled && mm_plan_z(c.pz.L);
             }
         }
         bx.threads = round64(tx);
@@ -1897,9 +1897,9 @@ template <typename T> struct BatchRunner : BatchRunnerBase {
         // per-system records and tile tables
         std::vector<BxDesc<T>> dx;
         std::vector<ByDesc<T>> dy;
-        std::vector<BzDesc<T>> dz;
+        std::vector<BzDesc<T>> dz, dzr;
         std::vector<B2Desc<T>> d2;
-        std::vector<int> tx_s, ty_s, tz_s, t2_s;
+        std::vector<int> tx_s, ty_s, tz_s, tzr_s, t2_s;
         auto add_tiles = [](std::vector<int> &t, int count, int sysi) {
             const int base = (int)t.size();
             t.insert(t.end(), (size_t)count, sysi);
@@ -1931,6 +1931,12 @@ template <typename T> struct BatchRunner : BatchRunnerBase {
                 by.o32 = by.o32 && o32;
                 dy.push_back(e);
                 BzDesc<T> f;
+                if (c.zreg_batch()) {
+                    t = mm_zreg_desc<T>(c, f, stop);
+                    f.tbase = add_tiles(tzr_s, t, (int)dzr.size());
+                    dzr.push_back(f);
+                    continue;
+                }
                 t = c.batch_z(f, bz.threads, lds, o32, stop);
                 f.tbase = add_tiles(tz_s, t, (int)dz.size());
                 bz.lds = std::max(bz.lds, lds);
@@ -1941,7 +1947,9 @@ template <typename T> struct BatchRunner : BatchRunnerBase {
         upload_pass(bx, dx, tx_s);
         if (any3d) {
             upload_pass(by, dy, ty_s);
-            upload_pass(bz, dz, tz_s);
+            if (!dz.empty()) upload_pass(bz, dz, tz_s);
+            bzr.threads = MM_ZREG_BATCH_THREADS;
+            if (!dzr.empty()) upload_pass(bzr, dzr, tzr_s);
         }
         if (any2d) upload_pass(b2, d2, t2_s);
         // stage launches, one per physics class present
@@ -2036,7 +2044,8 @@ template <typename T> struct BatchRunner : BatchRunnerBase {
         for (int st = 0; st < ns; ++st) {
             if (any3d) {
                 mm_batch_yfwd<T>(by, s);
-                mm_batch_zmi<T>(bz, s);
+                if (bz.ntiles) mm_batch_zmi<T>(bz, s);
+                if (bzr.ntiles) mm_batch_zreg<T>(bzr, s);
                 mm_batch_yinv<T>(by, s);
             }
             if (any2d) mm_batch_ymi2d<T>(b2, s);

@@ -53,3 +53,25 @@ def test_periodic_z_lines_stay_whole(nz, precision, tol):
     # a periodic axis has no zero half: its lines must not take the form that reads half
     H, ref = field((10, 6, nz), nz, precision, (False, False, True))
     assert rel_err(H, ref) < tol
+
+
+@pytest.mark.parametrize("precision", ["fp64", "fp32"])
+@pytest.mark.parametrize("layers", [(2, 3, 4), (2, 5, 4, 9), (5, 12)])
+def test_batch_of_short_z_lines(layers, precision, monkeypatch):
+    # register and LDS lines in one batch: every member as it steps alone
+    # (in the forms the batch takes: LDS beyond 8 points), bit for bit
+    from micromagnum_amd.solver import Ensemble, Stepper
+    kw = dict(delta=(2e-9, 2.5e-9, 3e-9), method="rkf45", precision=precision, Ms=8e5, alpha=0.5, A=1.3e-11)
+    specs = [dict(kw, shape=(33 + 7 * i, 18 + i, nz)) for i, nz in enumerate(layers)]
+    Ms = [random_unit_field(s["shape"], i) * 8e5 for i, s in enumerate(specs)]
+    monkeypatch.setenv("MM_BATCH_LAUNCH", "1")
+    ens = Ensemble(specs)
+    for i, M in enumerate(Ms):
+        ens.set_m(i, M)
+    ens.run(5)
+    for i, s in enumerate(specs):
+        monkeypatch.setenv("MM_FFT_GENERIC", "1" if layers[i] > 4 else "0")
+        st = Stepper(s["shape"], N=ens.specs[i].N, **{k: v for k, v in s.items() if k != "shape"})
+        st.set_m(Ms[i])
+        st.run(5)
+        assert np.array_equal(ens.get_m(i), st.get_m()), i
