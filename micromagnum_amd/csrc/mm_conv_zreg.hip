@@ -6,7 +6,7 @@
 // loads in flight, not for memory.  Here nothing is exchanged between threads:
 // every read of a thread is issued at its start, the rest is arithmetic, so
 // the pass is bound by the spectra's traffic.  200x200x5 FP64 (12 points): 27
-// -> 13 us, 58 MB.  Registers set the limit: 3 L complex values and the
+// -> 14 us, 58 MB.  Registers set the limit: 3 L complex values and the
 // kernel entries take 103 / 158 / 204 VGPRs at 8 / 12 / 16 points in FP32 and
 // 204 / 312 at 8 / 12 in FP64 (4, 3, 2 and 2, 1 waves per SIMD).
 #include "mm_conv.h"
