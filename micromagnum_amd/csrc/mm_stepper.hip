@@ -500,6 +500,9 @@ template <typename T> struct Stepper : public StepperBase {
     void download(double *dst, const T *src, size_t cnt)
     {
         if (cnt * sizeof(double) >= Readback<T>::MIN_BYTES) {
+            // the pieces serve one read at a time: a second thread that reads
+            // the same stepper waits
+            std::lock_guard<std::mutex> lk(readback_mu);
             if (!readback) readback.reset(new Readback<T>());
             if (readback->run(dst, src, cnt, s)) return;
         }
@@ -508,6 +511,7 @@ template <typename T> struct Stepper : public StepperBase {
         MM_HIP(hipMemcpyAsync(dst, dbuf, sizeof(double) * cnt, hipMemcpyDeviceToHost, s));
         MM_HIP(hipStreamSynchronize(s));
     }
+    std::mutex readback_mu;
     std::unique_ptr<Readback<T>> readback;
 
     bool own_stream = true;
