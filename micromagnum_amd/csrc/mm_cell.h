@@ -120,17 +120,31 @@ __device__ __forceinline__ V3<T> exchange_cell(const MeshDev &m, int x, int y, i
     return v3<T>(f * s.x / ms_i, f * s.y / ms_i, f * s.z / ms_i);
 }
 
-// exchange_cell for callers that hold the reciprocals of Ms: inv(j) is 1/Ms of
-// cell j, 0 where Ms is 0.  All neighbours load without branches, in one batch (a direction
-// without a neighbour reads the cell itself, whose difference is an exact
-// zero), and the divisions by Ms are products with inv: with a branch and
-// three divisions per neighbour the compiler waited for each neighbour's
-// loads in turn (200x200x5 FP64, per-cell Ms: inner stages 34.6 -> 32.8 us,
-// the final stage 32.9 -> 27.0 us).
-template <typename T, typename INV>
-__device__ __forceinline__ V3<T> exchange_cell_inv(const MeshDev &m, int x, int y, int z, size_t i, size_t n, T wx, T wy,
-                                               T wz, T coef, INV inv, const T *__restrict__ A,
-                                               const T *__restrict__ M)
+// v / d from r = 1 / d (rounded): the product, corrected by its own remainder
+// (Markstein's final step of a division), which rounds as v / d does.  The
+// same v and d give the same bits, so differences of equal quotients are exact
+// zeros; the bare product v r carries r's error, and its difference to another
+// one is contracted to a single rounding and is not zero.
+template <typename T> __device__ __forceinline__ T quotient(T v, T d, T r)
+{
+    const T u = v * r;
+    return fma(fma(-u, d, v), r, u);
+}
+
+// exchange_cell with the neighbours' loads in one batch and one division per
+// neighbour: a direction without a neighbour reads the cell itself and adds an
+// exact zero, neighbours with Ms == 0 are masked, and the terms are
+// exchange_cell's in its order.  With a branch and three divisions per
+// neighbour the compiler waited for each neighbour's loads in turn.  RKF45
+// step of a disk with per-cell Ms, MI355X, three divisions per neighbour ->
+// one: 200x200x5 FP32 279 -> 273 us, FP64 391 -> 388; 300x300x1 FP32 229 ->
+// 225, FP64 256 -> 254.  A branch to exchange_cell for an Ms so small that
+// 1 / Ms overflows cost 2 to 5 % of the step (the LLG factor alpha / Ms of such
+// a cell overflows as well).
+template <typename T>
+__device__ __forceinline__ V3<T> exchange_cell_batch(const MeshDev &m, int x, int y, int z, size_t i, size_t n, T wx,
+                                                     T wy, T wz, T coef, const T *__restrict__ Ms,
+                                                     const T *__restrict__ A, const T *__restrict__ M, T ms_i)
 {
     const long li = (long)i, sy = m.nx, sz = (long)m.nx * m.ny;
     long j[6];
@@ -140,27 +154,31 @@ __device__ __forceinline__ V3<T> exchange_cell_inv(const MeshDev &m, int x, int 
     j[3] = y < m.ny - 1 ? li + sy : (m.py ? li - sy * (m.ny - 1) : li);
     j[4] = z > 0 ? li - sz : (m.pz ? li + sz * (m.nz - 1) : li);
     j[5] = z < m.nz - 1 ? li + sz : (m.pz ? li - sz * (m.nz - 1) : li);
-    T a[6][3], r[6];
+    T a[6][3], ms[6];
 #pragma unroll
     for (int q = 0; q < 6; ++q) {
-        r[q] = inv(j[q]);
+        ms[q] = Ms[j[q]];
         a[q][0] = M[j[q]];
         a[q][1] = M[n + j[q]];
         a[q][2] = M[2 * n + j[q]];
     }
-    const T ri = inv(li);
-    const V3<T> mi = v3<T>(M[i] * ri, M[n + i] * ri, M[2 * n + i] * ri);
-    const T f = coef * A[i] * ri;
+    const T ri = (T)1 / ms_i;
+    const V3<T> mi = v3<T>(quotient(M[i], ms_i, ri), quotient(M[n + i], ms_i, ri), quotient(M[2 * n + i], ms_i, ri));
     const T w[6] = {wx, wx, wy, wy, wz, wz};
     V3<T> s = v3<T>(0, 0, 0);
 #pragma unroll
     for (int q = 0; q < 6; ++q) {
-        const bool on = r[q] != (T)0;
-        s.x += on ? (a[q][0] * r[q] - mi.x) * w[q] : (T)0;
-        s.y += on ? (a[q][1] * r[q] - mi.y) * w[q] : (T)0;
-        s.z += on ? (a[q][2] * r[q] - mi.z) * w[q] : (T)0;
+        const bool on = ms[q] != (T)0;
+        const T r = (T)1 / ms[q];
+        const T tx = s.x + (quotient(a[q][0], ms[q], r) - mi.x) * w[q];
+        const T ty = s.y + (quotient(a[q][1], ms[q], r) - mi.y) * w[q];
+        const T tz = s.z + (quotient(a[q][2], ms[q], r) - mi.z) * w[q];
+        s.x = on ? tx : s.x;
+        s.y = on ? ty : s.y;
+        s.z = on ? tz : s.z;
     }
-    return v3<T>(f * s.x, f * s.y, f * s.z);
+    const T f = coef * A[i];
+    return v3<T>(f * s.x / ms_i, f * s.y / ms_i, f * s.z / ms_i);
 }
 
 // uniaxial anisotropy: anisotropy_cpu.cpp:29-73

@@ -72,7 +72,6 @@ template <typename T> struct SysDev {
     T dx, dy, dz;
     T wx, wy, wz, coef_ex, mu0, cm2mu0, mu_b, e_charge;
     Param<T> Ms, A, f1, f2, alpha, kuni, kcub, P, xi;
-    const T *iMs;  // 1/Ms per cell, 0 where Ms is 0 (exchange with per-cell Ms/A)
     VParam<T> axis1, axis2, j;
     int has_exch, has_uni, has_cub, has_zee, has_stt, do_precess;
     T hext[3];
@@ -382,8 +381,8 @@ __device__ __forceinline__ void stage_cell(const SysDev<T> &S, const StageDev<T>
         } else {
             he = S.exch_uniform
                      ? exchange_cell_uniform<T>(S.m, x, y, z, i, n, S.wx, S.wy, S.wz, S.exch_f, Y)
-                     : exchange_cell_inv<T>(S.m, x, y, z, i, n, S.wx, S.wy, S.wz, S.coef_ex,
-                                        [&](long j) { return gfield(S.iMs)[j]; }, gfield(S.A.p), Y);
+                     : exchange_cell_batch<T>(S.m, x, y, z, i, n, S.wx, S.wy, S.wz, S.coef_ex, gfield(S.Ms.p),
+                                              gfield(S.A.p), Y, ms);
         }
         if constexpr (GEN == GEN_CUB) {
             // rounded before the sum, as GEN_ALL has it (there the field comes

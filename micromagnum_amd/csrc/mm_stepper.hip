@@ -591,15 +591,7 @@ template <typename T> struct Stepper : public StepperBase {
             upload(dp, d.A_host, n);
             sys.A.p = dp;
             sys.exch_uniform = sys.Ms_uniform && sys.Ms_u != 0.0 && all_equal(d.A_host, n);
-            if (sys.exch_uniform) {
-                sys.exch_f = (T)(2.0 * d.A_host[0] / (mu0 * sys.Ms_u * sys.Ms_u));
-            } else {
-                std::vector<double> r(n);
-                for (size_t i = 0; i < n; ++i) r[i] = d.Ms_host[i] != 0.0 ? 1.0 / d.Ms_host[i] : 0.0;
-                T *ip = dalloc(n);
-                upload(ip, r.data(), n);
-                sys.iMs = ip;
-            }
+            if (sys.exch_uniform) sys.exch_f = (T)(2.0 * d.A_host[0] / (mu0 * sys.Ms_u * sys.Ms_u));
         }
         sys.has_uni = d.k_uni_host != nullptr;
         sys.has_cub = d.k_cub_host != nullptr;
