@@ -26,18 +26,16 @@
 #include <algorithm>
 #include <chrono>
 #include <cmath>
-#include <condition_variable>
 #include <cstddef>
 #include <cstdint>
 #include <cstring>
 #include <map>
 #include <memory>
 #include <mutex>
-#include <system_error>
-#include <thread>
 #include <vector>
 
 #include "mm_stage.h"
+#include "mm_readback.h"
 
 // Relaxation rule on the state the attempt started from; true: stop there
 // (the attempt is discarded).  MM_RELAX_DMDT compares scaled_abs_max(dM/dt,
@@ -303,128 +301,6 @@ static bool all_equal(const double *a, size_t n)
     return true;
 }
 
-// Large device arrays of T to host doubles: pieces go through a few pinned
-// buffers in the state's own precision, and host threads widen (or copy) each
-// piece into the caller's array while the next ones are on their way.  A
-// pageable copy of doubles is staged by the runtime on one thread; that took
-// 18.8 ms for 512x512x32 (FP32 and FP64), 5.0 for 1024x1024x2 and 1.4 for
-// 256x256x16, this takes 4.9 / 7.4, 1.5 / 2.2 and 0.5 / 0.85 ms.
-template <typename T> struct Readback {
-    // of doubles: 200x200x8 (7.7 MB) reads in 0.47 ms either way, 256x256x6
-    // (9.4 MB) in 0.27 / 0.45 ms instead of 0.55
-    static constexpr size_t MIN_BYTES = (size_t)8 << 20;
-    static constexpr size_t PIECE = ((size_t)2 << 20) / sizeof(T);
-    static constexpr int NBUF = 4, NTHR = 8;
-    T *buf[NBUF] = {};
-    hipEvent_t ev[NBUF] = {};
-
-    Readback()
-    {
-        try {
-            for (int b = 0; b < NBUF; ++b) {
-                MM_HIP(hipHostMalloc((void **)&buf[b], PIECE * sizeof(T), hipHostMallocDefault));
-                MM_HIP(hipEventCreateWithFlags(&ev[b], hipEventDisableTiming));
-            }
-        } catch (...) {
-            release();
-            throw;
-        }
-    }
-    ~Readback() { release(); }
-    Readback(const Readback &) = delete;
-    void release()
-    {
-        for (int b = 0; b < NBUF; ++b) {
-            if (ev[b]) (void)hipEventDestroy(ev[b]);
-            if (buf[b]) (void)hipHostFree(buf[b]);
-            ev[b] = nullptr;
-            buf[b] = nullptr;
-        }
-    }
-
-    // false: the host gave no thread, nothing was read
-    bool run(double *dst, const T *src, size_t cnt, hipStream_t s)
-    {
-        const size_t np = (cnt + PIECE - 1) / PIECE;
-        std::mutex mu;
-        std::condition_variable cv;
-        size_t landed = 0;          // pieces in their buffers
-        bool quit = false;
-        int nthr = 0;               // set before the first piece lands
-        std::vector<int> done(np, 0);  // threads finished with a piece
-        std::vector<std::thread> thr;
-        auto work = [&](int t) {
-            for (size_t i = 0; i < np; ++i) {
-                {
-                    std::unique_lock<std::mutex> lk(mu);
-                    cv.wait(lk, [&] { return quit || landed > i; });
-                    if (landed <= i) return;
-                }
-                const size_t n = std::min(PIECE, cnt - i * PIECE);
-                const size_t a = n * t / nthr, e = n * (t + 1) / nthr;
-                const T *in = buf[i % NBUF];
-                double *out = dst + i * PIECE;
-                for (size_t j = a; j < e; ++j) out[j] = (double)in[j];
-                {
-                    std::lock_guard<std::mutex> lk(mu);
-                    if (++done[i] == nthr) cv.notify_all();
-                }
-            }
-        };
-        // every exit ends and joins the threads, and no copy into the buffers
-        // is left in flight
-        struct Join {
-            std::mutex &mu;
-            std::condition_variable &cv;
-            bool &quit;
-            std::vector<std::thread> &thr;
-            hipStream_t s;
-            ~Join()
-            {
-                {
-                    std::lock_guard<std::mutex> lk(mu);
-                    quit = true;
-                }
-                cv.notify_all();
-                for (std::thread &t : thr) t.join();
-                (void)hipStreamSynchronize(s);
-            }
-        } join{mu, cv, quit, thr, s};
-        thr.reserve(NTHR);
-        try {
-            for (int t = 0; t < NTHR; ++t) thr.emplace_back(work, t);
-        } catch (const std::system_error &) {
-            if (thr.empty()) return false;  // with fewer threads it goes on
-        }
-        nthr = (int)thr.size();
-        auto issue = [&](size_t i) {
-            const size_t n = std::min(PIECE, cnt - i * PIECE);
-            MM_HIP(hipMemcpyAsync(buf[i % NBUF], src + i * PIECE, n * sizeof(T), hipMemcpyDeviceToHost, s));
-            MM_HIP(hipEventRecord(ev[i % NBUF], s));
-        };
-        for (size_t i = 0; i < std::min<size_t>(np, NBUF); ++i) issue(i);
-        for (size_t i = 0; i < np; ++i) {
-            MM_HIP(hipEventSynchronize(ev[i % NBUF]));
-            {
-                std::lock_guard<std::mutex> lk(mu);
-                landed = i + 1;
-            }
-            cv.notify_all();
-            // the buffer of piece i + NBUF - 1 is piece i - 1's: refill it
-            // once that is through
-            if (i >= 1 && i - 1 + NBUF < np) {
-                std::unique_lock<std::mutex> lk(mu);
-                cv.wait(lk, [&] { return done[i - 1] == nthr; });
-                lk.unlock();
-                issue(i - 1 + NBUF);
-            }
-        }
-        std::unique_lock<std::mutex> lk(mu);
-        cv.wait(lk, [&] { return done[np - 1] == nthr; });
-        return true;
-    }
-};
-
 template <typename T> struct Stepper : public StepperBase {
     mm_system_desc_t d;
     size_t n = 0;
@@ -499,20 +375,13 @@ template <typename T> struct Stepper : public StepperBase {
 
     void download(double *dst, const T *src, size_t cnt)
     {
-        if (cnt * sizeof(double) >= Readback<T>::MIN_BYTES) {
-            // the pieces serve one read at a time: a second thread that reads
-            // the same stepper waits
-            std::lock_guard<std::mutex> lk(readback_mu);
-            if (!readback) readback.reset(new Readback<T>());
-            if (readback->run(dst, src, cnt, s)) return;
-        }
+        if (cnt * sizeof(double) >= Readback::MIN_BYTES && reader.read(dst, src, cnt, s)) return;
         hipLaunchKernelGGL(k_cast_out<T>, dim3(1024), dim3(256), 0, s, cnt, src, dbuf);
         MM_HIP(hipGetLastError());
         MM_HIP(hipMemcpyAsync(dst, dbuf, sizeof(double) * cnt, hipMemcpyDeviceToHost, s));
         MM_HIP(hipStreamSynchronize(s));
     }
-    std::mutex readback_mu;
-    std::unique_ptr<Readback<T>> readback;
+    StateReader reader;
 
     bool own_stream = true;
 
