@@ -149,14 +149,28 @@ __device__ __forceinline__ unsigned udiv(unsigned n, unsigned d, unsigned m)
     return d == 1 ? n : (m ? __umulhi(n, m) : n / d);
 }
 
-// Fourier kernel times spectrum of one point; k: xx, xy, xz, yy, yz, zz
+// Fourier kernel times spectrum of one point; k: xx, xy, xz, yy, yz, zz.  The
+// roundings are spelled out, as those of the DFTs.
 template <typename T>
 __device__ __forceinline__ void mult3(C2<T> &mx, C2<T> &my, C2<T> &mz, const T k[6])
 {
+    auto row = [](T a, T x, T b, T y, T c, T z) { return fma(c, z, fma(a, x, b * y)); };
     const C2<T> x = mx, y = my, z = mz;
-    mx = cmk<T>(k[0] * x.x + k[1] * y.x + k[2] * z.x, k[0] * x.y + k[1] * y.y + k[2] * z.y);
-    my = cmk<T>(k[1] * x.x + k[3] * y.x + k[4] * z.x, k[1] * x.y + k[3] * y.y + k[4] * z.y);
-    mz = cmk<T>(k[2] * x.x + k[4] * y.x + k[5] * z.x, k[2] * x.y + k[4] * y.y + k[5] * z.y);
+    mx = cmk<T>(row(k[0], x.x, k[1], y.x, k[2], z.x), row(k[0], x.y, k[1], y.y, k[2], z.y));
+    my = cmk<T>(row(k[1], x.x, k[3], y.x, k[4], z.x), row(k[1], x.y, k[3], y.y, k[4], z.y));
+    mz = cmk<T>(row(k[2], x.x, k[4], y.x, k[5], z.x), row(k[2], x.y, k[4], y.y, k[5], z.y));
+}
+
+// ... at the point mirrored in z of the one k belongs to: xz and yz change sign
+template <typename T>
+__device__ __forceinline__ void mult3_mirror(C2<T> &mx, C2<T> &my, C2<T> &mz, const T k[6])
+{
+    auto row = [](T a, T x, T b, T y, T c, T z) { return fma(-c, z, fma(a, x, b * y)); };
+    auto last = [](T a, T x, T b, T y, T c, T z) { return fma(c, z, fma(-b, y, -(a * x))); };
+    const C2<T> x = mx, y = my, z = mz;
+    mx = cmk<T>(row(k[0], x.x, k[1], y.x, k[2], z.x), row(k[0], x.y, k[1], y.y, k[2], z.y));
+    my = cmk<T>(row(k[1], x.x, k[3], y.x, k[4], z.x), row(k[1], x.y, k[3], y.y, k[4], z.y));
+    mz = cmk<T>(last(k[2], x.x, k[4], y.x, k[5], z.x), last(k[2], x.y, k[4], y.y, k[5], z.y));
 }
 
 static inline int floor_pow2(int v) { return v < 1 ? 1 : 1 << (31 - __builtin_clz((unsigned)v)); }
@@ -323,8 +337,9 @@ struct ConvImpl {
                          (L == 16 && sizeof(T) == 4 && cells >= 65536);
         return len && !g.is2d && !fft_generic && g.nz <= (L + 1) / 2 && cells * sizeof(C2<T>) < (1ull << 32);
     }
-    // ... and of a batched launch, whose kernel holds the lines of one pass
-    // (4 and 8 points, 2 to 4 layers), for which both forms give the same bits
+    // ... and of a batched launch, whose kernel holds the lines of one pass (4
+    // and 8 points, 2 to 4 layers).  Both forms give the same bits at every
+    // length, so that a member is a single stepper bit for bit.
     bool zreg_batch() const { return zreg() && (g.Pz == 4 || g.Pz == 8); }
     // threads per workgroup this system's passes need at least
     int batch_threads_x() const { return px.tline; }

@@ -392,16 +392,12 @@ __device__ __forceinline__ void zmi_body(C2<T> *__restrict__ S2, const T *__rest
         const int e = threadIdx.x + j * blockDim.x;
         const int col = e & (tk - 1), kzf = e >> ltk, kx = kx0 + col;
         if (e < nitems && kx < Hx) {
-            T k[6] = {kk[j][0], sy * kk[j][1], kk[j][2], kk[j][3], sy * kk[j][4], kk[j][5]};
+            const T k[6] = {kk[j][0], sy * kk[j][1], kk[j][2], kk[j][3], sy * kk[j][4], kk[j][5]};
             C2<T> *l0 = sm + (size_t)(0 * tk + col) * LP, *l1 = sm + (size_t)(1 * tk + col) * LP,
                   *l2 = sm + (size_t)(2 * tk + col) * LP;
             mult3<T>(l0[sk<SK>(kzf)], l1[sk<SK>(kzf)], l2[sk<SK>(kzf)], k);
             const int kz2 = L - kzf;
-            if (kzf > 0 && kz2 != kzf) {
-                k[2] = -k[2];
-                k[4] = -k[4];
-                mult3<T>(l0[sk<SK>(kz2)], l1[sk<SK>(kz2)], l2[sk<SK>(kz2)], k);
-            }
+            if (kzf > 0 && kz2 != kzf) mult3_mirror<T>(l0[sk<SK>(kz2)], l1[sk<SK>(kz2)], l2[sk<SK>(kz2)], k);
         }
     }
     __syncthreads();

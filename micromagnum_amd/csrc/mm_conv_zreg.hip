@@ -12,56 +12,9 @@
 #include "mm_conv.h"
 #include "mm_cell.h"
 
-// Size-R DFTs with every rounding spelled out as the LDS form's compiled code
-// has it, so that both forms give the same bits: a product that enters a sum
-// and a difference is fused into both, except in the last pass of the inverse
-// (SPLIT), where the LDS form's sums sit in the blocks of its guarded stores
-// and the product is rounded first.
-template <typename T, bool SPLIT> __device__ __forceinline__ void addsub(T e, T c, T x, T &sum, T &dif)
-{
-    if constexpr (SPLIT) {
-#pragma clang fp contract(off)
-        const T p = c * x;
-        sum = e + p;
-        dif = e - p;
-    } else {
-        sum = fma(c, x, e);
-        dif = fma(-c, x, e);
-    }
-}
-
-template <typename T, bool INV, bool SPLIT> __device__ __forceinline__ void dft3_reg(C2<T> *v)
-{
-    const T c = (T)-0.5;
-    const T s = INV ? (T)0.86602540378443864676372317075293618347140262690519
-                    : (T)-0.86602540378443864676372317075293618347140262690519;
-    const C2<T> t = cadd<T>(v[1], v[2]), d = csub<T>(v[1], v[2]);
-    const C2<T> m = cmk<T>(fma(c, t.x, v[0].x), fma(c, t.y, v[0].y));
-    v[0] = cadd<T>(v[0], t);
-    addsub<T, SPLIT>(m.x, -s, d.y, v[1].x, v[2].x);
-    addsub<T, SPLIT>(m.y, s, d.x, v[1].y, v[2].y);
-}
-
-template <typename T, bool INV, bool SPLIT> __device__ __forceinline__ void dft8_reg(C2<T> *v)
-{
-    C2<T> e[4] = {v[0], v[2], v[4], v[6]};
-    C2<T> o[4] = {v[1], v[3], v[5], v[7]};
-    dft4<T, INV>(e);
-    dft4<T, INV>(o);
-    const T h = (T)0.70710678118654752440084436210484903928483593768847;
-    const C2<T> o2 = cmul_mi<T, INV>(o[2]);
-    v[0] = cadd<T>(e[0], o[0]);
-    v[4] = csub<T>(e[0], o[0]);
-    addsub<T, SPLIT>(e[1].x, h, INV ? o[1].x - o[1].y : o[1].x + o[1].y, v[1].x, v[5].x);
-    addsub<T, SPLIT>(e[1].y, h, INV ? o[1].x + o[1].y : o[1].y - o[1].x, v[1].y, v[5].y);
-    v[2] = cadd<T>(e[2], o2);
-    v[6] = csub<T>(e[2], o2);
-    addsub<T, SPLIT>(e[3].x, INV ? -h : h, INV ? o[3].x + o[3].y : o[3].y - o[3].x, v[3].x, v[7].x);
-    addsub<T, SPLIT>(e[3].y, INV ? h : -h, INV ? o[3].x - o[3].y : o[3].x + o[3].y, v[3].y, v[7].y);
-}
-
-// The transform of a line in one thread's registers: the passes and twiddles
-// of fft_line, no LDS, no barriers.  tw is the plan's per-pass table in global
+// The transform of a line in one thread's registers: the passes, twiddles and
+// roundings of fft_line (SPLIT as its last inverse pass, which stores), no
+// LDS, no barriers.  tw is the plan's per-pass table in global
 // memory; its indices are constants and its base is uniform, so the twiddles
 // come in by scalar loads.
 template <typename T, bool INV, int LC, int PS = 0, int NS = 1>
@@ -79,15 +32,9 @@ __device__ __forceinline__ void fft_reg(C2<T> (&v)[LC], const C2<T> *__restrict_
 #pragma unroll
             for (int r = 0; r < R; ++r) {
                 u[r] = v[b + r * nb];
-                if (r > 0 && k > 0) {
-                    C2<T> w = tw[F::toff(PS) + (r - 1) * NS + k];
-                    if (INV) w.y = -w.y;
-                    u[r] = cmul<T>(u[r], w);
-                }
+                if (r > 0 && k > 0) u[r] = cmul_tw<T, INV>(u[r], tw[F::toff(PS) + (r - 1) * NS + k]);
             }
-            if constexpr (R == 8) dft8_reg<T, INV, SPLIT>(u);
-            else if constexpr (R == 3) dft3_reg<T, INV, SPLIT>(u);
-            else dftR<R, T, INV>(u);
+            dftR<R, T, INV, SPLIT>(u);
 #pragma unroll
             for (int r = 0; r < R; ++r) o[(b / NS) * NS * R + k + r * NS] = u[r];
         }
@@ -146,13 +93,9 @@ __device__ __forceinline__ void zmir_body(C2<T> *__restrict__ S2, const T *__res
     }
 #pragma unroll
     for (int kz = 0; kz <= LC / 2; ++kz) {
-        T k[6] = {kk[kz][0], sy * kk[kz][1], kk[kz][2], kk[kz][3], sy * kk[kz][4], kk[kz][5]};
+        const T k[6] = {kk[kz][0], sy * kk[kz][1], kk[kz][2], kk[kz][3], sy * kk[kz][4], kk[kz][5]};
         mult3<T>(v[0][kz], v[1][kz], v[2][kz], k);
-        if (kz > 0 && LC - kz != kz) {
-            k[2] = -k[2];
-            k[4] = -k[4];
-            mult3<T>(v[0][LC - kz], v[1][LC - kz], v[2][LC - kz], k);
-        }
+        if (kz > 0 && LC - kz != kz) mult3_mirror<T>(v[0][LC - kz], v[1][LC - kz], v[2][LC - kz], k);
     }
 #pragma unroll
     for (int c = 0; c < 3; ++c) {

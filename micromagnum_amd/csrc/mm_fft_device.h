@@ -111,6 +111,34 @@ template <typename T, int LC = 0> __device__ __forceinline__ void load_twiddles(
 template <int R> struct Log2R { static const int value = R == 8 ? 3 : (R == 4 ? 2 : 1); };
 
 // ---- size-R DFTs on registers --------------------------------------------
+// Every rounding is spelled out: which product of a sum is fused is left to
+// the compiler otherwise, and it chose differently in different kernels of one
+// length, so a field depended on the kernel that computed it.  With these,
+// every form of a transform (compiled or runtime plan, LDS or registers,
+// single or batched) gives the same bits.
+
+// a times the twiddle w (INV: its conjugate)
+template <typename T, bool INV> __device__ __forceinline__ C2<T> cmul_tw(C2<T> a, C2<T> w)
+{
+#pragma clang fp contract(off)
+    return INV ? cmk<T>(fma(w.x, a.x, w.y * a.y), fma(w.x, a.y, -(w.y * a.x)))
+               : cmk<T>(fma(w.x, a.x, -(w.y * a.y)), fma(w.x, a.y, w.y * a.x));
+}
+
+// sum = e + c x, dif = e - c x; SPLIT: the product is rounded first
+template <typename T, bool SPLIT> __device__ __forceinline__ void addsub(T e, T c, T x, T &sum, T &dif)
+{
+#pragma clang fp contract(off)
+    if constexpr (SPLIT) {
+        const T p = c * x;
+        sum = e + p;
+        dif = e - p;
+    } else {
+        sum = fma(c, x, e);
+        dif = fma(-c, x, e);
+    }
+}
+
 template <typename T, bool INV> __device__ __forceinline__ void dft2(C2<T> *v)
 {
     const C2<T> a = v[0], b = v[1];
@@ -128,45 +156,41 @@ template <typename T, bool INV> __device__ __forceinline__ void dft4(C2<T> *v)
     v[3] = csub<T>(t1, t3);
 }
 
-template <typename T, bool INV> __device__ __forceinline__ void dft8(C2<T> *v)
+template <typename T, bool INV, bool SPLIT> __device__ __forceinline__ void dft8(C2<T> *v)
 {
     C2<T> e[4] = {v[0], v[2], v[4], v[6]};
     C2<T> o[4] = {v[1], v[3], v[5], v[7]};
     dft4<T, INV>(e);
     dft4<T, INV>(o);
     const T h = (T)0.70710678118654752440084436210484903928483593768847;
-    // o[k] *= W8^k
-    const C2<T> o1 = INV ? cmk<T>(h * (o[1].x - o[1].y), h * (o[1].x + o[1].y))
-                         : cmk<T>(h * (o[1].x + o[1].y), h * (o[1].y - o[1].x));
+    // e[k] +- o[k] W8^k
     const C2<T> o2 = cmul_mi<T, INV>(o[2]);
-    const C2<T> o3 = INV ? cmk<T>(-h * (o[3].x + o[3].y), h * (o[3].x - o[3].y))
-                         : cmk<T>(h * (o[3].y - o[3].x), -h * (o[3].x + o[3].y));
     v[0] = cadd<T>(e[0], o[0]);
     v[4] = csub<T>(e[0], o[0]);
-    v[1] = cadd<T>(e[1], o1);
-    v[5] = csub<T>(e[1], o1);
+    addsub<T, SPLIT>(e[1].x, h, INV ? o[1].x - o[1].y : o[1].x + o[1].y, v[1].x, v[5].x);
+    addsub<T, SPLIT>(e[1].y, h, INV ? o[1].x + o[1].y : o[1].y - o[1].x, v[1].y, v[5].y);
     v[2] = cadd<T>(e[2], o2);
     v[6] = csub<T>(e[2], o2);
-    v[3] = cadd<T>(e[3], o3);
-    v[7] = csub<T>(e[3], o3);
+    addsub<T, SPLIT>(e[3].x, INV ? -h : h, INV ? o[3].x + o[3].y : o[3].y - o[3].x, v[3].x, v[7].x);
+    addsub<T, SPLIT>(e[3].y, INV ? h : -h, INV ? o[3].x - o[3].y : o[3].x + o[3].y, v[3].y, v[7].y);
 }
 
-template <typename T, bool INV> __device__ __forceinline__ void dft3(C2<T> *v)
+template <typename T, bool INV, bool SPLIT> __device__ __forceinline__ void dft3(C2<T> *v)
 {
     const T c = (T)-0.5;
     const T s = INV ? (T)0.86602540378443864676372317075293618347140262690519
                     : (T)-0.86602540378443864676372317075293618347140262690519;
     const C2<T> t = cadd<T>(v[1], v[2]), d = csub<T>(v[1], v[2]);
-    const C2<T> m = cmk<T>(v[0].x + c * t.x, v[0].y + c * t.y);
-    // i*s*d
-    const C2<T> isd = cmk<T>(-s * d.y, s * d.x);
+    const C2<T> m = cmk<T>(fma(c, t.x, v[0].x), fma(c, t.y, v[0].y));
     v[0] = cadd<T>(v[0], t);
-    v[1] = cadd<T>(m, isd);
-    v[2] = csub<T>(m, isd);
+    // m +- i s d
+    addsub<T, SPLIT>(m.x, -s, d.y, v[1].x, v[2].x);
+    addsub<T, SPLIT>(m.y, s, d.x, v[1].y, v[2].y);
 }
 
 template <typename T, bool INV> __device__ __forceinline__ void dft5(C2<T> *v)
 {
+#pragma clang fp contract(off)
     const T c1 = (T)0.30901699437494742410229341718281905886436044959787;   // cos(2pi/5)
     const T c2 = (T)-0.80901699437494742410229341718281905886436044959787;  // cos(4pi/5)
     const T s1 = (T)0.95105651629515357211643933337938214340569863412575;   // sin(2pi/5)
@@ -175,12 +199,10 @@ template <typename T, bool INV> __device__ __forceinline__ void dft5(C2<T> *v)
     const C2<T> b1 = cadd<T>(v[1], v[4]), d1 = csub<T>(v[1], v[4]);
     const C2<T> b2 = cadd<T>(v[2], v[3]), d2 = csub<T>(v[2], v[3]);
     const C2<T> a0 = v[0];
-    const C2<T> m1 = cmk<T>(a0.x + c1 * b1.x + c2 * b2.x, a0.y + c1 * b1.y + c2 * b2.y);
-    const C2<T> m2 = cmk<T>(a0.x + c2 * b1.x + c1 * b2.x, a0.y + c2 * b1.y + c1 * b2.y);
-    // which product of a sum is the fused one is spelled out: left to the
-    // compiler it differed between kernels of one length
+    const C2<T> m1 = cmk<T>(fma(c2, b2.x, fma(c1, b1.x, a0.x)), fma(c2, b2.y, fma(c1, b1.y, a0.y)));
+    const C2<T> m2 = cmk<T>(fma(c1, b2.x, fma(c2, b1.x, a0.x)), fma(c1, b2.y, fma(c2, b1.y, a0.y)));
     const C2<T> n1 = cmk<T>(sg * fma(s2, d2.x, s1 * d1.x), sg * fma(s2, d2.y, s1 * d1.y)); // times i below
-    const C2<T> n2 = cmk<T>(sg * (s2 * d1.x - s1 * d2.x), sg * (s2 * d1.y - s1 * d2.y));
+    const C2<T> n2 = cmk<T>(sg * fma(s2, d1.x, -(s1 * d2.x)), sg * fma(s2, d1.y, -(s1 * d2.y)));
     v[0] = cmk<T>(a0.x + b1.x + b2.x, a0.y + b1.y + b2.y);
     v[1] = cmk<T>(m1.x - n1.y, m1.y + n1.x);
     v[4] = cmk<T>(m1.x + n1.y, m1.y - n1.x);
@@ -188,13 +210,17 @@ template <typename T, bool INV> __device__ __forceinline__ void dft5(C2<T> *v)
     v[3] = cmk<T>(m2.x + n2.y, m2.y - n2.x);
 }
 
-template <int R, typename T, bool INV> __device__ __forceinline__ void dftR(C2<T> *v)
+// SPLIT: the radix-3 and radix-8 sums round their products first.  The last
+// pass of an inverse transform that stores its outputs takes it: those stores
+// are guarded one by one, each output is formed inside its guard, and fields
+// keep the bits they have had there.
+template <int R, typename T, bool INV, bool SPLIT = false> __device__ __forceinline__ void dftR(C2<T> *v)
 {
     if constexpr (R == 2) dft2<T, INV>(v);
-    else if constexpr (R == 3) dft3<T, INV>(v);
+    else if constexpr (R == 3) dft3<T, INV, SPLIT>(v);
     else if constexpr (R == 4) dft4<T, INV>(v);
     else if constexpr (R == 5) dft5<T, INV>(v);
-    else dft8<T, INV>(v);
+    else dft8<T, INV, SPLIT>(v);
 }
 
 // Maximum butterflies per thread and pass for radix R when a line of length
@@ -228,11 +254,7 @@ __device__ __forceinline__ void fft_pass(C2<T> *line, const C2<T> *__restrict__ 
             const int k = P2 ? (b & (Ns - 1)) : b % Ns;
             if (Ns > 1) {
 #pragma unroll
-                for (int r = 1; r < R; ++r) {
-                    C2<T> w = tw[toff + (r - 1) * Ns + k];
-                    if (INV) w.y = -w.y;
-                    v[q][r] = cmul<T>(v[q][r], w);
-                }
+                for (int r = 1; r < R; ++r) v[q][r] = cmul_tw<T, INV>(v[q][r], tw[toff + (r - 1) * Ns + k]);
             }
             dftR<R, T, INV>(v[q]);
             const int base = P2 ? (((b >> lNs) << (lNs + Log2R<R>::value)) + k) : (b / Ns) * Ns * R + k;
@@ -342,13 +364,9 @@ __device__ __forceinline__ void fft_pass_io(C2<T> *lineG, LineMap g, C2<T> *line
             const int k = P2 ? (b & (Ns - 1)) : b % Ns;
             if (Ns > 1) {
 #pragma unroll
-                for (int r = 1; r < R; ++r) {
-                    C2<T> w = tw[toff + (r - 1) * Ns + k];
-                    if (INV) w.y = -w.y;
-                    v[q][r] = cmul<T>(v[q][r], w);
-                }
+                for (int r = 1; r < R; ++r) v[q][r] = cmul_tw<T, INV>(v[q][r], tw[toff + (r - 1) * Ns + k]);
             }
-            dftR<R, T, INV>(v[q]);
+            dftR<R, T, INV, INV && STOUT>(v[q]);
             const int base = P2 ? (((b >> lNs) << (lNs + Log2R<R>::value)) + k) : (b / Ns) * Ns * R + k;
 #pragma unroll
             for (int r = 0; r < R; ++r) {
