@@ -65,9 +65,9 @@ struct FftPlanHost {
 };
 
 // Calls f(std::integral_constant<int, LC>()) with the kernel instantiation for
-// lines of length L: LC = L for powers of two 2..2048 (unless `generic`),
-// MM_LC_ANY (MM_LC_Z for the z pass) for the other compiled lengths, else 0,
-// the runtime plan.
+// lines of length L: LC = L for powers of two 2..2048, MM_LC_ANY (MM_LC_Z for
+// the z pass) for the other compiled lengths, else and with `generic` 0, the
+// runtime plan.
 template <int ANY = MM_LC_ANY, typename F> void mm_with_len(int L, bool generic, F &&f)
 {
     if (!generic) {
@@ -77,9 +77,12 @@ template <int ANY = MM_LC_ANY, typename F> void mm_with_len(int L, bool generic,
 #undef MM_FFT_X
         default: break;
         }
+        if (mm_plan_id(L) > 0 && (ANY != MM_LC_Z || mm_plan_z(L))) {
+            f(std::integral_constant<int, ANY>());
+            return;
+        }
     }
-    if (mm_plan_id(L) > 0 && (ANY != MM_LC_Z || mm_plan_z(L))) f(std::integral_constant<int, ANY>());
-    else f(std::integral_constant<int, 0>());
+    f(std::integral_constant<int, 0>());
 }
 
 bool mm_is_smooth(int n);                  // n has no prime factor > 5

@@ -566,14 +566,14 @@ void ConvImpl<T>::init(const double *N_host, int nx, int ny, int nz, int ex, int
     px.build(g.Px);
     py.build(g.Py);
     pz.build(g.Pz);
-    if (!mm_plan_z(g.Pz)) pz.no_compiled();
+    // MM_FFT_GENERIC=1: runtime FFT plans for every length, single and batched
+    // (tests compare them with the compiled plans)
+    fft_generic = env_int("MM_FFT_GENERIC", 0) != 0;
+    if (fft_generic)
+        for (FftPlanHost *p : {&px, &py, &pz}) p->no_compiled();
+    else if (!mm_plan_z(g.Pz))
+        pz.no_compiled();
     ln = mm_choose_launch(g, px, py, pz, sizeof(C2<T>));
-    // MM_FFT_GENERIC=1: runtime FFT plans for every length (tests compare
-    // them with the compile-time plans)
-    {
-        const char *e = std::getenv("MM_FFT_GENERIC");
-        fft_generic = e && std::atoi(e) != 0;
-    }
     // MM_WIDE_INDEX=1: the general forms of the index arithmetic (integer
     // division, 64-bit element addressing) that grids beyond the 32-bit
     // ranges take, for any grid (tests compare both; the results are equal)

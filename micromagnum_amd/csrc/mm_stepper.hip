@@ -1752,7 +1752,7 @@ template <typename T> struct BatchRunner : BatchRunnerBase {
                 b2.compiled = b2.compiled && c.py.id > 0;
             } else {
                 by.compiled = by.compiled && c.py.id > 0;
-                if (!c.zreg_batch()) bz.compiled = bz.compiled && mm_plan_z(c.pz.L);
+                if (!c.zreg_batch()) bz.compiled = bz.compiled && c.pz.id > 0;
             }
         }
         bx.threads = round64(tx);
