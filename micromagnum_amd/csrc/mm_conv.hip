@@ -5,6 +5,7 @@
 #include "mm_cell.h"
 
 #include <algorithm>
+#include <climits>
 #include <cmath>
 #include <cstdlib>
 #include <cstring>
@@ -94,14 +95,17 @@ bool mm_is_smooth(int n)
 int mm_fft_size_for(int n, int given)
 {
     if (n == 1) return 1;
-    if (given < 2 * n - 1) {
+    if (given < 2ll * n - 1) {
         MM_REQUIRE(given == n, "tensor size along an axis must be the mesh size (periodic) or >= 2n-1 (open)");
         MM_REQUIRE(mm_is_smooth(n), "a periodic axis needs a mesh size of the form 2^a 3^b 5^c");
         return n;
     }
     if (given % 2 == 0 && mm_is_smooth(given)) return given;
-    int p = 2 * n - 1;
-    while (!(p % 2 == 0 && mm_is_smooth(p))) ++p;
+    int p = 2 * n - 1;  // fits: given is no smaller
+    while (!(p % 2 == 0 && mm_is_smooth(p))) {
+        MM_REQUIRE(p < INT_MAX, "no transform length for this mesh size");
+        ++p;
+    }
     return p;
 }
 
