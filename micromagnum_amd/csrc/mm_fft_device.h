@@ -490,7 +490,8 @@ constexpr bool mm_plan_z(int L)
 }
 
 // passes of a length 2^a 3^b 5^c: radix 8 while it divides, then one 4 or 2,
-// then the fives, then the threes; n = 0 if there is another factor
+// then the fives, then the threes; n = 0 if there is another factor.  n counts
+// all of them; of more than 16 (no plan takes so many) the first 16 are kept.
 struct FftRadices {
     int n, r[16];
 };
@@ -499,13 +500,20 @@ constexpr FftRadices mm_plan_radices(int L)
     FftRadices f = {0, {}};
     int m = L, twos = 0;
     for (; m % 2 == 0; m /= 2) ++twos;
-    for (; twos >= 3; twos -= 3) f.r[f.n++] = 8;
-    if (twos) f.r[f.n++] = 1 << twos;
-    for (; m % 5 == 0; m /= 5) f.r[f.n++] = 5;
-    for (; m % 3 == 0; m /= 3) f.r[f.n++] = 3;
+    for (; twos >= 3; twos -= 3, ++f.n)
+        if (f.n < 16) f.r[f.n] = 8;
+    if (twos) {
+        if (f.n < 16) f.r[f.n] = 1 << twos;
+        ++f.n;
+    }
+    for (; m % 5 == 0; m /= 5, ++f.n)
+        if (f.n < 16) f.r[f.n] = 5;
+    for (; m % 3 == 0; m /= 3, ++f.n)
+        if (f.n < 16) f.r[f.n] = 3;
     if (m != 1) f.n = 0;
     return f;
 }
+static_assert(mm_plan_radices(1162261467).n == 19, "3^19, the most factors of an int");
 // Threads per line of a compiled length.  Powers of two: L/8.  Else the count
 // that wastes the fewest thread slots over the passes (each deals its butterflies
 // out in rounds of that many), counting a butterfly's arithmetic and element

@@ -7,7 +7,8 @@ import pytest
 from micromagnum_amd import _lib
 
 
-@pytest.mark.parametrize("n,message", [(5 ** 13, "passes")])
+@pytest.mark.parametrize("n,message", [(3 ** 9, "passes"), (3 ** 16, "passes"), (3 ** 17, "passes"), (3 ** 19, "passes"),
+                                       (2 * 3 ** 17, "passes"), (5 ** 13, "passes")])
 def test_lengths_with_too_many_factors(n, message):
     # periodic along x, whose tensor has the mesh's own size; it is not read
     L = _lib.load()
