@@ -518,8 +518,9 @@ static_assert(mm_plan_radices(1162261467).n == 19, "3^19, the most factors of an
 // that wastes the fewest thread slots over the passes (each deals its butterflies
 // out in rounds of that many), counting a butterfly's arithmetic and element
 // accesses, times a tenth more per round (the line's latency); equal counts
-// go to the wider one.  At least a twelfth of the
-// line, which the z pass's kernel items need.
+// go to the wider one.  At least L/12, which the z pass's kernel items need, and
+// L/8, for which the kernels that run a plan in a loop have registers (they
+// take a compiled plan's count where a batch falls back to them).
 constexpr int mm_plan_tline(int L)
 {
     if ((L & (L - 1)) == 0) return L > MM_FFT_EPT ? L / MM_FFT_EPT : 1;
@@ -527,7 +528,7 @@ constexpr int mm_plan_tline(int L)
     int most = 1, best = 1;
     long cost = -1;
     for (int p = 0; p < f.n; ++p) most = L / f.r[p] > most ? L / f.r[p] : most;
-    for (int t = (L / 2 + 6) / 6; t <= most || cost < 0; ++t) {
+    for (int t = (L + MM_FFT_EPT - 1) / MM_FFT_EPT; t <= most || cost < 0; ++t) {
         long c = 0, rounds = 10;
         for (int p = 0; p < f.n; ++p) {
             const int R = f.r[p], nb = L / R, mb = (nb + t - 1) / t;
@@ -549,6 +550,7 @@ template <int LC> struct FftLen {
     static constexpr int npass = f.n;
     static constexpr bool p2 = (LC & (LC - 1)) == 0;
     static constexpr int tline = mm_plan_tline(LC);
+    static_assert(tline * MM_FFT_EPT >= LC && 6 * tline >= LC / 2 + 1, "too few threads per line");
     static constexpr int radix(int ps) { return f.r[ps]; }
     // butterflies per thread of pass ps
     static constexpr int mb(int ps) { return (LC / f.r[ps] + tline - 1) / tline; }
