@@ -38,6 +38,14 @@ struct FftPlanHost {
         id = 0;
         tline = tline_loop(L);
     }
+    // the narrow plan of a length that has one (y passes)
+    void narrow()
+    {
+        if (const int n = mm_plan_id(L, true)) {
+            id = n;
+            tline = mm_plan_tline(L, true);
+        }
+    }
     template <typename T> FftPlanDev dev_loop() const
     {
         FftPlanDev d = dev<T>();
@@ -66,8 +74,8 @@ struct FftPlanHost {
 
 // Calls f(std::integral_constant<int, LC>()) with the kernel instantiation for
 // lines of length L: LC = L for powers of two 2..2048, MM_LC_ANY (MM_LC_Z for
-// the z pass) for the other compiled lengths, else and with `generic` 0, the
-// runtime plan.
+// the z pass, MM_LC_Y for the y passes) for the other compiled lengths, else
+// and with `generic` 0, the runtime plan.
 template <int ANY = MM_LC_ANY, typename F> void mm_with_len(int L, bool generic, F &&f)
 {
     if (!generic) {
@@ -376,6 +384,7 @@ struct mm_conv {
 
 void mm_lds_attr_once();
 int mm_max_lds_bytes();
+int mm_num_cus();  // of the current device
 
 // Launch shapes of a mesh (0: not set, the built-in choice applies): x lines
 // per workgroup, kx columns per workgroup of the y and z passes, rows per

@@ -125,6 +125,14 @@ int mm_max_lds_bytes()
     return g_max_lds;
 }
 
+int mm_num_cus()
+{
+    int dev = 0, n = 0;
+    MM_HIP(hipGetDevice(&dev));
+    MM_HIP(hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev));
+    return n;
+}
+
 // ---------------------------------------------------------------------------
 // launch-shape table ("wisdom")
 // ---------------------------------------------------------------------------

@@ -573,6 +573,19 @@ void ConvImpl<T>::init(const double *N_host, int nx, int ny, int nz, int ex, int
         for (FftPlanHost *p : {&px, &py, &pz}) p->no_compiled();
     else if (!mm_plan_z(g.Pz))
         pz.no_compiled();
+    // The narrow y plans once the wide ones, whose tiles hold one column (2-D)
+    // or two to four (3-D), fill the chip: there the row segments count, and
+    // fewer workgroups finish sooner with more threads to a line.  Field, wide
+    // -> narrow, MI355X: 256x450x1 (900 points, 257 workgroups) FP64 55.0 ->
+    // 42.5 us, FP32 32.1 -> 33.0; 450x450x8 FP64 403 -> 358, FP32 196 -> 164;
+    // 500x500x1 FP64 80.5 -> 72.5; 270x270x8 FP64 136 -> 131, FP32 81.4 ->
+    // 83.8; below, 64x450x1 (65 workgroups) FP32 22.7 -> 27.1, 64x270x1 FP64
+    // 21.9 -> 23.9.
+    {
+        const int cols = floor_pow2(1024 / ((g.is2d ? 3 : 1) * py.tline));
+        const size_t wgs = (size_t)((g.Hx + cols - 1) / cols) * (g.is2d ? 1 : 3 * nz);
+        if (!fft_generic && wgs >= (size_t)mm_num_cus()) py.narrow();
+    }
     ln = mm_choose_launch(g, px, py, pz, sizeof(C2<T>));
     // MM_WIDE_INDEX=1: the general forms of the index arithmetic (integer
     // division, 64-bit element addressing) that grids beyond the 32-bit
@@ -741,7 +754,7 @@ template <typename T> void ConvImpl<T>::spectral(hipStream_t s)
     if (g.is2d) {
         const int tk = ln.tk_y;
         const size_t sh = lines_lds<MM_SKEW_Y>(3 * tk, py.L, cs);
-        mm_with_len(py.L, fft_generic, [&](auto lc) {
+        mm_with_len<MM_LC_Y>(py.L, fft_generic, [&](auto lc) {
             hipLaunchKernelGGL((k_ymi2d<T, decltype(lc)::value>), dim3((g.Hx + tk - 1) / tk), dim3(3 * tk * py.tline),
                                sh, s, S1, kern, plane, g.Hx, g.Hp, g.Hy2, g.ny, py.dev<T>(), tk);
         });
@@ -760,7 +773,7 @@ template <typename T> void ConvImpl<T>::spectral(hipStream_t s)
         hipLaunchKernelGGL((k_yfwd_pr<T>), dim3((g.Hx + tkp - 1) / tkp, g.nz, 3), dim3(tkp * pyh.tline), shyp, s, S1, S2,
                            g.Hx, g.Hp, g.ny, g.nz, pyh.dev<T>(), (const C2<T> *)py.plain<T>(), tkp);
     } else {
-        mm_with_len(py.L, fft_generic, [&](auto lc) {
+        mm_with_len<MM_LC_Y>(py.L, fft_generic, [&](auto lc) {
             const unsigned ntx = (unsigned)((g.Hx + tk - 1) / tk), nb = ntx * g.nz * 3;
             if (y_o32)
                 hipLaunchKernelGGL((k_yfwd<T, decltype(lc)::value, true>), dim3(ntx, g.nz, 3), dim3(tk * py.tline), shy,
@@ -799,7 +812,7 @@ template <typename T> void ConvImpl<T>::spectral(hipStream_t s)
         hipLaunchKernelGGL((k_yinv_pr<T>), dim3((g.Hx + tkp - 1) / tkp, g.nz, 3), dim3(tkp * pyh.tline), shyp, s, S2, S1,
                            g.Hx, g.Hp, g.ny, g.nz, pyh.dev<T>(), (const C2<T> *)py.plain<T>(), tkp);
     } else {
-        mm_with_len(py.L, fft_generic, [&](auto lc) {
+        mm_with_len<MM_LC_Y>(py.L, fft_generic, [&](auto lc) {
             const unsigned ntx = (unsigned)((g.Hx + tk - 1) / tk), nb = ntx * g.nz * 3;
             if (y_o32)
                 hipLaunchKernelGGL((k_yinv<T, decltype(lc)::value, true>), dim3(ntx, g.nz, 3), dim3(tk * py.tline), shy,
@@ -1007,7 +1020,7 @@ template <typename T> void mm_batch_xfwd(const BatchPass &bp, hipStream_t s)
 }
 template <typename T, bool INV> static void batch_y_pass(const BatchPass &bp, hipStream_t s)
 {
-    batch_kind<MM_LC_ANY>(bp, [&](auto lc, auto o32) {
+    batch_kind<MM_LC_Y>(bp, [&](auto lc, auto o32) {
         hipLaunchKernelGGL((kb_y<T, INV, decltype(lc)::value, decltype(o32)::value>), dim3(bp.ntiles),
                            dim3(bp.threads), bp.lds, s, (const ByDesc<T> *)bp.desc, (const int *)bp.tsys);
     });
@@ -1025,7 +1038,7 @@ template <typename T> void mm_batch_zmi(const BatchPass &bp, hipStream_t s)
 }
 template <typename T> void mm_batch_ymi2d(const BatchPass &bp, hipStream_t s)
 {
-    batch_kind<MM_LC_ANY>(bp, [&](auto lc, auto) {
+    batch_kind<MM_LC_Y>(bp, [&](auto lc, auto) {
         hipLaunchKernelGGL((kb_ymi2d<T, decltype(lc)::value>), dim3(bp.ntiles), dim3(bp.threads), bp.lds, s,
                            (const B2Desc<T> *)bp.desc, (const int *)bp.tsys);
     });

@@ -470,12 +470,19 @@ __device__ __forceinline__ void fft_line_p2(const FftPlanDev &p, const C2<T> *tw
     X(360) X(384) X(400) X(432) X(450) X(480) X(486) X(500) X(540) X(576) X(600) X(640) X(648) X(720) X(750)      \
     X(768) X(800) X(900) X(960) X(1000)
 
+// lengths whose threads per line leave one or two columns to a y tile; the y
+// passes hold them a second time, with fewer threads (narrow)
+#define MM_FFT_NARROW(X) X(540) X(648) X(900) X(1000)
+
 // number of a compiled length in the tables, 0 if it is in none
-constexpr int mm_plan_id(int L)
+constexpr int mm_plan_id(int L, bool narrow = false)
 {
     int id = 0, found = 0;
-#define MM_FFT_X(N) ++id; if (L == N) found = id;
+#define MM_FFT_X(N) ++id; if (L == N && !narrow) found = id;
     MM_FFT_POW2(MM_FFT_X) MM_FFT_MIXED_Z(MM_FFT_X) MM_FFT_MIXED_XY(MM_FFT_X)
+#undef MM_FFT_X
+#define MM_FFT_X(N) ++id; if (L == N && narrow) found = id;
+    MM_FFT_NARROW(MM_FFT_X)
 #undef MM_FFT_X
     return found;
 }
@@ -520,14 +527,16 @@ static_assert(mm_plan_radices(1162261467).n == 19, "3^19, the most factors of an
 // accesses, times a tenth more per round (the line's latency); equal counts
 // go to the wider one.  At least L/12, which the z pass's kernel items need, and
 // L/8, for which the kernels that run a plan in a loop have registers (they
-// take a compiled plan's count where a batch falls back to them).
-constexpr int mm_plan_tline(int L)
+// take a compiled plan's count where a batch falls back to them).  Narrow: at
+// most a sixth of a workgroup, two columns of the 2-D y pass.
+constexpr int mm_plan_tline(int L, bool narrow = false)
 {
     if ((L & (L - 1)) == 0) return L > MM_FFT_EPT ? L / MM_FFT_EPT : 1;
     const FftRadices f = mm_plan_radices(L);
     int most = 1, best = 1;
     long cost = -1;
     for (int p = 0; p < f.n; ++p) most = L / f.r[p] > most ? L / f.r[p] : most;
+    if (narrow && most > 1024 / 6) most = 1024 / 6;
     for (int t = (L + MM_FFT_EPT - 1) / MM_FFT_EPT; t <= most || cost < 0; ++t) {
         long c = 0, rounds = 10;
         for (int p = 0; p < f.n; ++p) {
@@ -544,12 +553,12 @@ constexpr int mm_plan_tline(int L)
     return best;
 }
 
-template <int LC> struct FftLen {
+template <int LC, bool NARROW = false> struct FftLen {
     static constexpr FftRadices f = mm_plan_radices(LC);
     static_assert(f.n > 0 && LC > 1, "no compiled plan of this length");
     static constexpr int npass = f.n;
     static constexpr bool p2 = (LC & (LC - 1)) == 0;
-    static constexpr int tline = mm_plan_tline(LC);
+    static constexpr int tline = mm_plan_tline(LC, NARROW);
     static_assert(tline * MM_FFT_EPT >= LC && 6 * tline >= LC / 2 + 1, "too few threads per line");
     static constexpr int radix(int ps) { return f.r[ps]; }
     // butterflies per thread of pass ps
@@ -569,10 +578,11 @@ template <int LC> struct FftLen {
 constexpr int mm_ilog2(int v) { return v <= 1 ? 0 : 1 + mm_ilog2(v >> 1); }
 
 // line length and threads per line of a kernel instantiated for LC (0: the
-// runtime plan p; MM_LC_ANY, MM_LC_Z: a compiled length selected at run time,
-// any or one of the z pass's)
+// runtime plan p; MM_LC_ANY, MM_LC_Z, MM_LC_Y: a compiled length selected at
+// run time, any, one of the z pass's, or any and the narrow ones)
 #define MM_LC_ANY (-1)
 #define MM_LC_Z (-2)
+#define MM_LC_Y (-3)
 template <int LC> struct PlanC {
     __device__ static constexpr int L(const FftPlanDev &) { return LC; }
     __device__ static constexpr int tline(const FftPlanDev &) { return FftLen<LC>::tline; }
@@ -584,19 +594,20 @@ struct PlanRun {
 template <> struct PlanC<0> : PlanRun {};
 template <> struct PlanC<MM_LC_ANY> : PlanRun {};
 template <> struct PlanC<MM_LC_Z> : PlanRun {};
+template <> struct PlanC<MM_LC_Y> : PlanRun {};
 
-template <typename T, bool INV, int LC, int PS, int NS, bool LDIN, bool STOUT, int SK, typename LD, typename ST,
+template <typename T, bool INV, int LC, bool NARROW, int PS, int NS, bool LDIN, bool STOUT, int SK, typename LD, typename ST,
           typename PF>
 __device__ __forceinline__ void fft_line_c(const C2<T> *tw, C2<T> *lineG, LineMap g, C2<T> *lineS, LineMap s_,
                                            LD &ld, ST &st, PF &pre)
 {
-    using F = FftLen<LC>;
+    using F = FftLen<LC, NARROW>;
     if constexpr (PS < F::npass) {
         constexpr int R = F::radix(PS);
         constexpr bool I = LDIN && PS == 0, O = STOUT && PS == F::npass - 1;
         fft_pass_io<R, F::mb(PS), T, INV, F::p2, I, O, SK, PS == 0>(lineG, g, lineS, s_, tw, LC, F::tline, NS,
                                                                     mm_ilog2(NS), F::toff(PS), ld, st, pre);
-        fft_line_c<T, INV, LC, PS + 1, NS * R, LDIN, STOUT, SK>(tw, lineG, g, lineS, s_, ld, st, pre);
+        fft_line_c<T, INV, LC, NARROW, PS + 1, NS * R, LDIN, STOUT, SK>(tw, lineG, g, lineS, s_, ld, st, pre);
     }
 }
 
@@ -614,10 +625,10 @@ __device__ __forceinline__ void fft_line(const FftPlanDev &p, const C2<T> *tw, C
                                          LineMap s_, LD ld, ST st, PF pre = PF())
 {
     if constexpr (LC > 0) {
-        fft_line_c<T, INV, LC, 0, 1, LDIN, STOUT, SK>(tw, lineG, g, lineS, s_, ld, st, pre);
+        fft_line_c<T, INV, LC, false, 0, 1, LDIN, STOUT, SK>(tw, lineG, g, lineS, s_, ld, st, pre);
     } else if constexpr (LC < 0) {
         // one workgroup runs one length: a uniform jump
-#define MM_FFT_X(N) case mm_plan_id(N): fft_line_c<T, INV, N, 0, 1, LDIN, STOUT, SK>(tw, lineG, g, lineS, s_, ld, st, pre); break;
+#define MM_FFT_X(N) case mm_plan_id(N): fft_line_c<T, INV, N, false, 0, 1, LDIN, STOUT, SK>(tw, lineG, g, lineS, s_, ld, st, pre); break;
         if constexpr (LC == MM_LC_Z) {
             switch (p.id) {
             MM_FFT_X(2) MM_FFT_X(4) MM_FFT_X(8) MM_FFT_X(16) MM_FFT_X(32) MM_FFT_X(64) MM_FFT_X(128)
@@ -629,6 +640,9 @@ __device__ __forceinline__ void fft_line(const FftPlanDev &p, const C2<T> *tw, C
             MM_FFT_POW2(MM_FFT_X)
             MM_FFT_MIXED_Z(MM_FFT_X)
             MM_FFT_MIXED_XY(MM_FFT_X)
+#undef MM_FFT_X
+#define MM_FFT_X(N) case mm_plan_id(N, true): if constexpr (LC == MM_LC_Y) fft_line_c<T, INV, N, true, 0, 1, LDIN, STOUT, SK>(tw, lineG, g, lineS, s_, ld, st, pre); break;
+            MM_FFT_NARROW(MM_FFT_X)
             default: break;
             }
         }

@@ -533,7 +533,7 @@ template <typename T> struct Stepper : public StepperBase {
                 // fewer workgroups than CUs (an ensemble's systems share the
                 // chip: they keep the fuller workgroups)
                 if (!ext)
-                    while (np > 1 && (d.ny * d.nz + 2 * np - 1) / (2 * np) < num_cus()) np = (np + 1) / 2;
+                    while (np > 1 && (d.ny * d.nz + 2 * np - 1) / (2 * np) < mm_num_cus()) np = (np + 1) / 2;
                 if (wshape.rpw > 0) np = std::max(1, wshape.rpw / 2);
                 if (const char *e = std::getenv("MM_RPW")) np = std::max(1, std::atoi(e) / 2);
                 // a tuned, imported or environment row count is cut to what one
@@ -577,7 +577,7 @@ template <typename T> struct Stepper : public StepperBase {
             // keep it so.  128x32x1 FP64: stage 16.1 -> 9.8 us with the
             // one-pair workgroups above; 150x90x14 FP32: 26.5 -> 17.8 us.
             if (!ext) {
-                const int wgs = (d.ny * d.nz + rpw - 1) / rpw, cus = num_cus();
+                const int wgs = (d.ny * d.nz + rpw - 1) / rpw, cus = mm_num_cus();
                 for (int t = std::min(1024, std::max(fft_threads, rpw * ((d.nx + 63) / 64 * 64))); t > threads; t -= 64)
                     if (stage_occupancy(t) * cus >= wgs) {
                         threads = t;
@@ -697,14 +697,6 @@ template <typename T> struct Stepper : public StepperBase {
         if (gen == GEN_ALL) return f(std::integral_constant<int, GEN_ALL>());
         if (gen == GEN_CUB) return f(std::integral_constant<int, GEN_CUB>());
         return f(std::integral_constant<int, GEN_NONE>());
-    }
-
-    static int num_cus()
-    {
-        int dev = 0, n = 0;
-        MM_HIP(hipGetDevice(&dev));
-        MM_HIP(hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev));
-        return n;
     }
 
     // workgroups of the stage kernel (this system's instantiation) that one
