@@ -38,13 +38,13 @@ struct FftPlanHost {
         id = 0;
         tline = tline_loop(L);
     }
-    // the narrow plan of a length that has one (y passes)
-    void narrow()
+    // the narrow plan of a length that has one (id 0 if not), on the same tables
+    FftPlanHost narrow() const
     {
-        if (const int n = mm_plan_id(L, true)) {
-            id = n;
-            tline = mm_plan_tline(L, true);
-        }
+        FftPlanHost n = *this;
+        n.id = mm_plan_id(L, true);
+        if (n.id > 0) n.tline = mm_plan_tline(L, true);
+        return n;
     }
     template <typename T> FftPlanDev dev_loop() const
     {
@@ -74,8 +74,8 @@ struct FftPlanHost {
 
 // Calls f(std::integral_constant<int, LC>()) with the kernel instantiation for
 // lines of length L: LC = L for powers of two 2..2048, MM_LC_ANY (MM_LC_Z for
-// the z pass, MM_LC_Y for the y passes) for the other compiled lengths, else
-// and with `generic` 0, the runtime plan.
+// the z pass) for the other compiled lengths, else and with `generic` 0, the
+// runtime plan.
 template <int ANY = MM_LC_ANY, typename F> void mm_with_len(int L, bool generic, F &&f)
 {
     if (!generic) {
@@ -304,6 +304,19 @@ struct ConvImpl {
     bool prune_y = false;
     bool wide = false;         // general index arithmetic only (MM_WIDE_INDEX)
     int tk_yp = 1;          // kx columns per WG of the pruned y transforms
+    // The y passes run py's narrow plan.  Single launches only: a batch's
+    // workgroups select their lengths in one kernel.
+    bool y_narrow = false;
+    FftPlanHost pyn;
+    int tk_yn = 1;
+    int tk_y() const { return y_narrow ? tk_yn : ln.tk_y; }
+    // the y passes address by 32-bit offsets (S2, 3 nz Py rows, is the larger
+    // of their two arrays)
+    bool y_offsets32() const
+    {
+        const size_t cs = sizeof(C2<T>);
+        return (size_t)g.Hp * cs < (1u << 24) && (size_t)3 * g.nz * g.Py * g.Hp * cs < (1ull << 32) && !wide;
+    }
     T *kern = nullptr;      // 6 real planes [e][kz<Hz2][ky<Hy2][kx<Hx], pitch Hp, scaled 1/(PxPyPz)
     C2<T> *S1 = nullptr;    // [c][z<nz][y<ny][kx<Hx], pitch Hp
     C2<T> *S2 = nullptr;    // [c][z<nz][ky<Py][kx<Hx], pitch Hp   (3-D only)
@@ -357,6 +370,11 @@ struct ConvImpl {
     int batch_threads_y() const { return (g.is2d ? 3 : 1) * py.tline; }
     int batch_threads_z() const { return 3 * pz.tline; }
 };
+
+// y passes of narrow plans (ConvImpl::y_narrow): 3-D forward and inverse, 2-D
+template <typename T> void mm_narrow_yfwd(const ConvImpl<T> &c, hipStream_t s);
+template <typename T> void mm_narrow_yinv(const ConvImpl<T> &c, hipStream_t s);
+template <typename T> void mm_narrow_ymi2d(const ConvImpl<T> &c, hipStream_t s);
 
 // z pass in registers (ConvImpl::zreg)
 template <typename T> void mm_zreg_pass(const ConvImpl<T> &c, hipStream_t s);

@@ -577,14 +577,16 @@ void ConvImpl<T>::init(const double *N_host, int nx, int ny, int nz, int ex, int
     // or two to four (3-D), fill the chip: there the row segments count, and
     // fewer workgroups finish sooner with more threads to a line.  Field, wide
     // -> narrow, MI355X: 256x450x1 (900 points, 257 workgroups) FP64 55.0 ->
-    // 42.5 us, FP32 32.1 -> 33.0; 450x450x8 FP64 403 -> 358, FP32 196 -> 164;
-    // 500x500x1 FP64 80.5 -> 72.5; 270x270x8 FP64 136 -> 131, FP32 81.4 ->
-    // 83.8; below, 64x450x1 (65 workgroups) FP32 22.7 -> 27.1, 64x270x1 FP64
+    // 41.7 us, FP32 33.0 -> 32.3; 450x450x8 FP64 401 -> 356, FP32 196 -> 162;
+    // 500x500x1 FP64 80.5 -> 70.2; 270x270x8 FP64 136 -> 129, FP32 81.4 ->
+    // 81.3; below, 64x450x1 (65 workgroups) FP32 22.7 -> 27.1, 64x270x1 FP64
     // 21.9 -> 23.9.
     {
         const int cols = floor_pow2(1024 / ((g.is2d ? 3 : 1) * py.tline));
         const size_t wgs = (size_t)((g.Hx + cols - 1) / cols) * (g.is2d ? 1 : 3 * nz);
-        if (!fft_generic && wgs >= (size_t)mm_num_cus()) py.narrow();
+        pyn = py.narrow();
+        y_narrow = !fft_generic && pyn.id > 0 && wgs >= (size_t)mm_num_cus();
+        if (y_narrow) tk_yn = mm_choose_launch(g, px, pyn, pz, sizeof(C2<T>)).tk_y;
     }
     ln = mm_choose_launch(g, px, py, pz, sizeof(C2<T>));
     // MM_WIDE_INDEX=1: the general forms of the index arithmetic (integer
@@ -754,7 +756,8 @@ template <typename T> void ConvImpl<T>::spectral(hipStream_t s)
     if (g.is2d) {
         const int tk = ln.tk_y;
         const size_t sh = lines_lds<MM_SKEW_Y>(3 * tk, py.L, cs);
-        mm_with_len<MM_LC_Y>(py.L, fft_generic, [&](auto lc) {
+        if (y_narrow) mm_narrow_ymi2d<T>(*this, s);
+        else mm_with_len(py.L, fft_generic, [&](auto lc) {
             hipLaunchKernelGGL((k_ymi2d<T, decltype(lc)::value>), dim3((g.Hx + tk - 1) / tk), dim3(3 * tk * py.tline),
                                sh, s, S1, kern, plane, g.Hx, g.Hp, g.Hy2, g.ny, py.dev<T>(), tk);
         });
@@ -764,16 +767,16 @@ template <typename T> void ConvImpl<T>::spectral(hipStream_t s)
     }
     const int tk = ln.tk_y;
     const size_t shy = lines_lds<MM_SKEW_Y>(tk, py.L, cs);
-    // S2 (3 nz Py rows) is the larger of the two arrays
-    const bool y_o32 =
-        (size_t)g.Hp * cs < (1u << 24) && (size_t)3 * g.nz * g.Py * g.Hp * cs < (1ull << 32) && !wide;
+    const bool y_o32 = y_offsets32();
     const int tkp = tk_yp;
     const size_t shyp = lines_lds<MM_SKEW_Y>(tkp, pyh.L, cs);
     if (prune_y) {
         hipLaunchKernelGGL((k_yfwd_pr<T>), dim3((g.Hx + tkp - 1) / tkp, g.nz, 3), dim3(tkp * pyh.tline), shyp, s, S1, S2,
                            g.Hx, g.Hp, g.ny, g.nz, pyh.dev<T>(), (const C2<T> *)py.plain<T>(), tkp);
+    } else if (y_narrow) {
+        mm_narrow_yfwd<T>(*this, s);
     } else {
-        mm_with_len<MM_LC_Y>(py.L, fft_generic, [&](auto lc) {
+        mm_with_len(py.L, fft_generic, [&](auto lc) {
             const unsigned ntx = (unsigned)((g.Hx + tk - 1) / tk), nb = ntx * g.nz * 3;
             if (y_o32)
                 hipLaunchKernelGGL((k_yfwd<T, decltype(lc)::value, true>), dim3(ntx, g.nz, 3), dim3(tk * py.tline), shy,
@@ -811,8 +814,10 @@ template <typename T> void ConvImpl<T>::spectral(hipStream_t s)
     if (prune_y) {
         hipLaunchKernelGGL((k_yinv_pr<T>), dim3((g.Hx + tkp - 1) / tkp, g.nz, 3), dim3(tkp * pyh.tline), shyp, s, S2, S1,
                            g.Hx, g.Hp, g.ny, g.nz, pyh.dev<T>(), (const C2<T> *)py.plain<T>(), tkp);
+    } else if (y_narrow) {
+        mm_narrow_yinv<T>(*this, s);
     } else {
-        mm_with_len<MM_LC_Y>(py.L, fft_generic, [&](auto lc) {
+        mm_with_len(py.L, fft_generic, [&](auto lc) {
             const unsigned ntx = (unsigned)((g.Hx + tk - 1) / tk), nb = ntx * g.nz * 3;
             if (y_o32)
                 hipLaunchKernelGGL((k_yinv<T, decltype(lc)::value, true>), dim3(ntx, g.nz, 3), dim3(tk * py.tline), shy,
@@ -1020,7 +1025,7 @@ template <typename T> void mm_batch_xfwd(const BatchPass &bp, hipStream_t s)
 }
 template <typename T, bool INV> static void batch_y_pass(const BatchPass &bp, hipStream_t s)
 {
-    batch_kind<MM_LC_Y>(bp, [&](auto lc, auto o32) {
+    batch_kind<MM_LC_ANY>(bp, [&](auto lc, auto o32) {
         hipLaunchKernelGGL((kb_y<T, INV, decltype(lc)::value, decltype(o32)::value>), dim3(bp.ntiles),
                            dim3(bp.threads), bp.lds, s, (const ByDesc<T> *)bp.desc, (const int *)bp.tsys);
     });
@@ -1038,7 +1043,7 @@ template <typename T> void mm_batch_zmi(const BatchPass &bp, hipStream_t s)
 }
 template <typename T> void mm_batch_ymi2d(const BatchPass &bp, hipStream_t s)
 {
-    batch_kind<MM_LC_Y>(bp, [&](auto lc, auto) {
+    batch_kind<MM_LC_ANY>(bp, [&](auto lc, auto) {
         hipLaunchKernelGGL((kb_ymi2d<T, decltype(lc)::value>), dim3(bp.ntiles), dim3(bp.threads), bp.lds, s,
                            (const B2Desc<T> *)bp.desc, (const int *)bp.tsys);
     });
@@ -1050,3 +1055,43 @@ template void mm_batch_yfwd<MM_CONV_T>(const BatchPass &, hipStream_t);
 template void mm_batch_yinv<MM_CONV_T>(const BatchPass &, hipStream_t);
 template void mm_batch_zmi<MM_CONV_T>(const BatchPass &, hipStream_t);
 template void mm_batch_ymi2d<MM_CONV_T>(const BatchPass &, hipStream_t);
+
+// y passes of narrow plans.  Behind everything else: between the other kernels
+// of this file they moved those, whose times hang on where their code lies
+// (150x90x14 FP32 y inverse 7.3 -> 7.8 us with the same code).
+template <typename T, bool INV> static void narrow_y(const ConvImpl<T> &c, hipStream_t s)
+{
+    const ConvGeom &g = c.g;
+    const int tk = c.tk_yn;
+    const size_t sh = lines_lds<MM_SKEW_Y>(tk, c.pyn.L, sizeof(C2<T>));
+    const unsigned ntx = (unsigned)((g.Hx + tk - 1) / tk), nb = ntx * g.nz * 3;
+    const dim3 grid(ntx, g.nz, 3), block(tk * c.pyn.tline);
+    const FftPlanDev p = c.pyn.template dev<T>();
+    const unsigned mx = mdiv(ntx, nb, c.wide), mz = mdiv((unsigned)g.nz, nb, c.wide);
+    auto go = [&](auto o32) {
+        constexpr bool O32 = decltype(o32)::value;
+        if constexpr (INV)
+            hipLaunchKernelGGL((k_yinv<T, MM_LC_NARROW, O32>), grid, block, sh, s, c.S2, c.S1, g.Hx, g.Hp, g.ny, g.nz,
+                               p, tk, c.xcd_remap, mx, mz);
+        else
+            hipLaunchKernelGGL((k_yfwd<T, MM_LC_NARROW, O32>), grid, block, sh, s, c.S1, c.S2, g.Hx, g.Hp, g.ny, g.nz,
+                               p, tk, c.xcd_remap, mx, mz);
+    };
+    if (c.y_offsets32()) go(std::true_type());
+    else go(std::false_type());
+    MM_HIP(hipGetLastError());
+}
+template <typename T> void mm_narrow_yfwd(const ConvImpl<T> &c, hipStream_t s) { narrow_y<T, false>(c, s); }
+template <typename T> void mm_narrow_yinv(const ConvImpl<T> &c, hipStream_t s) { narrow_y<T, true>(c, s); }
+template <typename T> void mm_narrow_ymi2d(const ConvImpl<T> &c, hipStream_t s)
+{
+    const ConvGeom &g = c.g;
+    const int tk = c.tk_yn;
+    hipLaunchKernelGGL((k_ymi2d<T, MM_LC_NARROW>), dim3((g.Hx + tk - 1) / tk), dim3(3 * tk * c.pyn.tline),
+                       lines_lds<MM_SKEW_Y>(3 * tk, c.pyn.L, sizeof(C2<T>)), s, c.S1, c.kern,
+                       (size_t)g.Hp * g.Hy2 * g.Hz2, g.Hx, g.Hp, g.Hy2, g.ny, c.pyn.template dev<T>(), tk);
+    MM_HIP(hipGetLastError());
+}
+template void mm_narrow_yfwd<MM_CONV_T>(const ConvImpl<MM_CONV_T> &, hipStream_t);
+template void mm_narrow_yinv<MM_CONV_T>(const ConvImpl<MM_CONV_T> &, hipStream_t);
+template void mm_narrow_ymi2d<MM_CONV_T>(const ConvImpl<MM_CONV_T> &, hipStream_t);

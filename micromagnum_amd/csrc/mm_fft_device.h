@@ -470,8 +470,10 @@ __device__ __forceinline__ void fft_line_p2(const FftPlanDev &p, const C2<T> *tw
     X(360) X(384) X(400) X(432) X(450) X(480) X(486) X(500) X(540) X(576) X(600) X(640) X(648) X(720) X(750)      \
     X(768) X(800) X(900) X(960) X(1000)
 
-// lengths whose threads per line leave one or two columns to a y tile; the y
-// passes hold them a second time, with fewer threads (narrow)
+// lengths whose threads per line leave one column to a 2-D y tile; the y passes
+// have kernels that hold these alone, with fewer threads (narrow).  In the
+// kernel of all mixed lengths they slowed the others (150x90x14 FP32, 180
+// points: y forward 8.0 -> 9.0 us, inverse 7.2 -> 7.7).
 #define MM_FFT_NARROW(X) X(540) X(648) X(900) X(1000)
 
 // number of a compiled length in the tables, 0 if it is in none
@@ -578,11 +580,11 @@ template <int LC, bool NARROW = false> struct FftLen {
 constexpr int mm_ilog2(int v) { return v <= 1 ? 0 : 1 + mm_ilog2(v >> 1); }
 
 // line length and threads per line of a kernel instantiated for LC (0: the
-// runtime plan p; MM_LC_ANY, MM_LC_Z, MM_LC_Y: a compiled length selected at
-// run time, any, one of the z pass's, or any and the narrow ones)
+// runtime plan p; MM_LC_ANY, MM_LC_Z, MM_LC_NARROW: a compiled length selected
+// at run time, any, one of the z pass's, or a narrow one)
 #define MM_LC_ANY (-1)
 #define MM_LC_Z (-2)
-#define MM_LC_Y (-3)
+#define MM_LC_NARROW (-3)
 template <int LC> struct PlanC {
     __device__ static constexpr int L(const FftPlanDev &) { return LC; }
     __device__ static constexpr int tline(const FftPlanDev &) { return FftLen<LC>::tline; }
@@ -594,7 +596,7 @@ struct PlanRun {
 template <> struct PlanC<0> : PlanRun {};
 template <> struct PlanC<MM_LC_ANY> : PlanRun {};
 template <> struct PlanC<MM_LC_Z> : PlanRun {};
-template <> struct PlanC<MM_LC_Y> : PlanRun {};
+template <> struct PlanC<MM_LC_NARROW> : PlanRun {};
 
 template <typename T, bool INV, int LC, bool NARROW, int PS, int NS, bool LDIN, bool STOUT, int SK, typename LD, typename ST,
           typename PF>
@@ -635,18 +637,23 @@ __device__ __forceinline__ void fft_line(const FftPlanDev &p, const C2<T> *tw, C
             MM_FFT_MIXED_Z(MM_FFT_X)
             default: break;
             }
-        } else {
+        } else if constexpr (LC == MM_LC_ANY) {
             switch (p.id) {
             MM_FFT_POW2(MM_FFT_X)
             MM_FFT_MIXED_Z(MM_FFT_X)
             MM_FFT_MIXED_XY(MM_FFT_X)
-#undef MM_FFT_X
-#define MM_FFT_X(N) case mm_plan_id(N, true): if constexpr (LC == MM_LC_Y) fft_line_c<T, INV, N, true, 0, 1, LDIN, STOUT, SK>(tw, lineG, g, lineS, s_, ld, st, pre); break;
-            MM_FFT_NARROW(MM_FFT_X)
             default: break;
             }
         }
 #undef MM_FFT_X
+        if constexpr (LC == MM_LC_NARROW) {
+#define MM_FFT_X(N) case mm_plan_id(N, true): fft_line_c<T, INV, N, true, 0, 1, LDIN, STOUT, SK>(tw, lineG, g, lineS, s_, ld, st, pre); break;
+            switch (p.id) {
+            MM_FFT_NARROW(MM_FFT_X)
+            default: break;
+            }
+#undef MM_FFT_X
+        }
     } else {
         if (p.pow2) fft_line_p2<T, INV, true, LDIN, STOUT, SK>(p, tw, lineG, g, lineS, s_, ld, st, pre);
         else fft_line_p2<T, INV, false, LDIN, STOUT, SK>(p, tw, lineG, g, lineS, s_, ld, st, pre);

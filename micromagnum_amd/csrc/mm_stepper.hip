@@ -1164,7 +1164,7 @@ template <typename T> struct Stepper : public StepperBase {
         MmShape r = {0, 0, 0, 0, 0};
         if (conv) {
             r.lpw_x = conv->ln.lpw_x;
-            r.tk_y = conv->ln.tk_y;
+            r.tk_y = conv->tk_y();
             r.tk_z = conv->ln.tk_z;
         }
         if (conv && !split_x) {
