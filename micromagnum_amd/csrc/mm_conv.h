@@ -353,6 +353,9 @@ struct ConvImpl {
     // 16 points it costs more than the barriers it saves.  FP64 lines of 16
     // points leave one wave per SIMD (200x200x8: 83.9 -> 87.7), 20 and more
     // likewise in FP32 (99x85x9: 29.7 -> 31.5, 256x256x16: 93.7 -> 105).
+    // Up to 12 points the mesh may be as small as it likes: 24x24x5 FP64 23.9
+    // -> 24.7, 40x30x5 25.2 -> 25.9, 64x64x5 26.0 -> 25.9, 100x100x5 33.8 ->
+    // 31.2 (launch-bound below), FP32 level there.
     bool zreg() const
     {
         const int L = g.Pz;

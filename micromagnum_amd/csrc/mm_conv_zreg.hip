@@ -14,9 +14,9 @@
 
 // The transform of a line in one thread's registers: the passes, twiddles and
 // roundings of fft_line (SPLIT as its last inverse pass, which stores), no
-// LDS, no barriers.  tw is the plan's per-pass table in global
-// memory; its indices are constants and its base is uniform, so the twiddles
-// come in by scalar loads.
+// LDS, no barriers.  tw is the plan's per-pass table in global memory; its
+// indices are constants and its base is uniform, so the twiddles come in by
+// scalar loads.
 template <typename T, bool INV, int LC, int PS = 0, int NS = 1>
 __device__ __forceinline__ void fft_reg(C2<T> (&v)[LC], const C2<T> *__restrict__ tw)
 {
@@ -44,7 +44,8 @@ __device__ __forceinline__ void fft_reg(C2<T> (&v)[LC], const C2<T> *__restrict_
     }
 }
 
-// One thread holds the z lines of the three components of one (kx, ky).  Threads run over the rows' whole pitch, so a
+// One thread holds the z lines of the three components of one (kx, ky).
+// Threads run over the rows' whole pitch, so a
 // wave's accesses are contiguous; (c, z) planes and kernel planes have uniform
 // bases and the thread's offset in a plane is one 32-bit value.  Needs
 // nz <= (LC + 1) / 2 (lines at least half zeros), so the upper half of a line
@@ -120,8 +121,12 @@ template <typename T> void mm_zreg_pass(const ConvImpl<T> &c, hipStream_t s)
     const ConvGeom &g = c.g;
     MM_REQUIRE(c.zreg(), "z pass has no register form of this line");
     const size_t plane = (size_t)g.Hp * g.Hy2 * g.Hz2, cells = (size_t)g.Py * g.Hp;
-    // below a workgroup of 256 per SIMD single waves spread evenly over the CUs
-    const unsigned bs = cells < 262144 ? 64u : 256u, nb = (unsigned)((cells + bs - 1) / bs);
+    // Workgroups of one wave spread evenly over the CUs; of four once there are
+    // enough of them, up to 8 points: longer FP64 lines leave one wave per SIMD,
+    // and a workgroup of four waits for a whole CU.  Field, 64 -> 256 threads:
+    // 1024x1024x2 FP32 202.9 -> 200.9 us, 512x512x4 FP64 173.8 -> 174.4;
+    // 512x512x5 FP64 207.6 -> 214.7, FP32 102.4 -> 103.1; 40x30x5 FP64 23.2 -> 24.0.
+    const unsigned bs = cells < 262144 || g.Pz > 8 ? 64u : 256u, nb = (unsigned)((cells + bs - 1) / bs);
     const unsigned mhp = mdiv((unsigned)g.Hp, (size_t)nb * bs, c.wide);
     const C2<T> *tw = (const C2<T> *)c.pz.template dev<T>().tw;
     switch (g.Pz) {

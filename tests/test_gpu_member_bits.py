@@ -39,3 +39,23 @@ def test_members_are_single_steppers(kind, precision):
         assert ens.stats(i) == st.stats(), members[i]
         st.close()
     ens.close()
+
+
+@pytest.mark.parametrize("precision", ["fp64", "fp32"])
+@pytest.mark.parametrize("shape,length", [((400, 330, 5), 12), ((400, 330, 3), 8), ((120, 90, 6), 12)])
+def test_register_lines_have_the_bits_of_the_others(shape, length, precision, monkeypatch):
+    # on both sides of the workgroup sizes' rule (2^18 columns)
+    from micromagnum_amd import magneto as mg
+    from micromagnum_amd.device import empty, to_device
+    N = mg.GenerateDemagTensor(*shape, 2e-9, 2.5e-9, 3e-9, device="gpu")
+    dt = np.float64 if precision == "fp64" else np.float32
+    M = to_device(random_unit_field(shape, 3) * 8e5, dt)
+    out = []
+    for generic in ("0", "1"):
+        monkeypatch.setenv("MM_FFT_GENERIC", generic)
+        conv = mg.SymmetricMatrixVectorConvolution_FFT(N, *shape, precision=precision)
+        assert conv.fft_size[2] == length
+        H = empty(M.shape, dt)
+        conv.execute(M, H)
+        out.append(H.numpy())
+    assert np.array_equal(out[0], out[1])
