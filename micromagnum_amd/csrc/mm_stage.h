@@ -693,6 +693,9 @@ __device__ __forceinline__ void stage_body(const SysDev<T> *__restrict__ Sp, con
     // the workgroup idle while it walks the rows one after another; the row
     // stays uniform per wave (scalar y, z and tile edges).  48 systems of
     // 32..256 cells per row, batched: stage 211 -> 162 us (MI355X, FP32).
+    // The loops step unsigned: with a signed step, which cannot wrap, the
+    // compiler turned the addresses of every array into induction variables of
+    // the x loop (FP32 77 -> 88 to 101 VGPRs, FP64 110 -> 128 and spilled).
     const int nwv = (int)(blockDim.x >> 6);
     const int wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const int rw = min(nwv, (nx + 63) >> 6), ngr = nwv / rw, grp = wv / rw;
@@ -705,7 +708,7 @@ __device__ __forceinline__ void stage_body(const SysDev<T> *__restrict__ Sp, con
         }
         const int gr = row0 + r;
         const int q = r >> 1, hi = r & 1;
-        for (int x = (int)threadIdx.x - grp * rw * 64; x < nx; x += rw * 64) {
+        for (int x = (int)(threadIdx.x - (unsigned)(grp * rw * 64)); x < nx; x = (int)((unsigned)x + (unsigned)(rw * 64))) {
             if (gr >= nrows) {
                 // the absent second row of a pair transforms as zeros
                 if (fused)
@@ -736,7 +739,7 @@ __device__ __forceinline__ void stage_body(const SysDev<T> *__restrict__ Sp, con
             const int lw = min(nwv, (L - nx + 63) >> 6), nlg = lw > 0 ? nwv / lw : 1, lg = lw > 0 ? wv / lw : 0;
             if (lg < nlg)
                 for (int l = lg; l < 3 * np; l += nlg)
-                    for (int x = nx + (int)threadIdx.x - lg * lw * 64; x < L; x += lw * 64)
+                    for (int x = (int)((unsigned)nx + threadIdx.x - (unsigned)(lg * lw * 64)); x < L; x = (int)((unsigned)x + (unsigned)(lw * 64)))
                         sm[(size_t)l * LP + sk<SK>(x)] = cmk<T>((T)0, (T)0);
         }
         __syncthreads();
@@ -761,7 +764,7 @@ __device__ __forceinline__ void stage_body(const SysDev<T> *__restrict__ Sp, con
             const bool has1 = gr0 + 1 < nrows;
             const C2<T> *ln = sm + (size_t)l * LP;
             C2<T> *d0 = gfield(G.fwd_S1) + ((size_t)c * nrows + gr0) * Hp;
-            for (int k = (int)threadIdx.x - lg * lw * 64; k < kh; k += lw * 64) {
+            for (int k = (int)(threadIdx.x - (unsigned)(lg * lw * 64)); k < kh; k = (int)((unsigned)k + (unsigned)(lw * 64))) {
                 const C2<T> zk = ln[sk<SK>(k)], zm = ln[sk<SK>(k == 0 ? 0 : L - k)];
                 d0[k] = cmk<T>((zk.x + zm.x) * (T)0.5, (zk.y - zm.y) * (T)0.5);
                 if (has1) d0[(size_t)Hp + k] = cmk<T>((zk.y + zm.y) * (T)0.5, (zm.x - zk.x) * (T)0.5);
@@ -836,9 +839,11 @@ __device__ __forceinline__ void stage_body(const SysDev<T> *__restrict__ Sp, con
 // that kernel needs 55-59 VGPRs and is held to 7 waves per SIMD by its 106
 // SGPRs; asking for 8 (SGPRs 78, the rest spilled to VGPR lanes, no
 // scratch) lets a CU hold 8 of its 256-thread workgroups, one round for
-// 256x256x16 cells: stage 32.4 -> 30.7 us (MI355X, same-run A/B).
+// 256x256x16 cells: stage 32.4 -> 30.7 us (MI355X, same-run A/B).  The other
+// FP32 kernels ask for 6 (80 VGPRs, no scratch; 81 without): 24 waves a CU,
+// two workgroups of 768 threads on 1024-cell rows with spin torque.
 template <typename T, bool EN, int LC, bool STT, int GEN, bool P1S = false>
-__global__ void __attribute__((amdgpu_waves_per_eu((P1S && sizeof(T) == 4) ? 8 : 1))) k_stage(const SysDev<T> *__restrict__ Sp, const StageDev<T> *__restrict__ Gp, StepCtl *ctl,
+__global__ void __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 ? (P1S ? 8 : (EN ? 1 : 6)) : 1))) k_stage(const SysDev<T> *__restrict__ Sp, const StageDev<T> *__restrict__ Gp, StepCtl *ctl,
                         const C2<T> *__restrict__ S1, FftPlanDev p, int Hx, int Hp, int rpw, int has_demag,
                         double *__restrict__ epart, const T *__restrict__ Hdem)
 {
