@@ -840,8 +840,9 @@ __device__ __forceinline__ void stage_body(const SysDev<T> *__restrict__ Sp, con
 // SGPRs; asking for 8 (SGPRs 78, the rest spilled to VGPR lanes, no
 // scratch) lets a CU hold 8 of its 256-thread workgroups, one round for
 // 256x256x16 cells: stage 32.4 -> 30.7 us (MI355X, same-run A/B).  The other
-// FP32 kernels ask for 6 (80 VGPRs, no scratch; 81 without): 24 waves a CU,
-// two workgroups of 768 threads on 1024-cell rows with spin torque.
+// FP32 kernels ask for 6 (80 VGPRs, 81 to 83 without; none to three spilled,
+// in spin torque with cubic anisotropy, all mixed lengths and runtime plans):
+// 24 waves a CU, two workgroups of 768 threads on 1024-cell rows.
 template <typename T, bool EN, int LC, bool STT, int GEN, bool P1S = false>
 __global__ void __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 ? (P1S ? 8 : (EN ? 1 : 6)) : 1))) k_stage(const SysDev<T> *__restrict__ Sp, const StageDev<T> *__restrict__ Gp, StepCtl *ctl,
                         const C2<T> *__restrict__ S1, FftPlanDev p, int Hx, int Hp, int rpw, int has_demag,
